@@ -12,7 +12,7 @@
 // 8 K-values with one 16-byte load; weights are pre-swizzled into per-lane
 // fragments so every wave reads them with one coalesced 1 KB load per tile.
 // The input-gradient pass is the same kernel over transposed, tap-flipped
-// weights; the weight-gradient pass stages 32-pixel chunks through LDS.
+// weights; the weight-gradient pass transposes pixel tiles through LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -154,113 +154,204 @@ __global__ __launch_bounds__(256) void k_conv(const bf16* __restrict__ in, int c
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient: dW[tap][ci][co] += sum_p dpre[p][co] * in[p + off(tap)][ci],
-// db[co] += sum_p dpre[p][co] (tap 4's blocks only). Grid: (tap, slice); each
-// block walks its slice of 32-pixel chunks (32 consecutive pixels in NHWC
-// order, the last chunk zero-padded), staging both operands in LDS, and its
-// four waves split the (co-tile, ci-tile) pairs, at most WG_MAX_PAIRS each.
-// Each block owns its slice's partial sums and stores them to its own row of
-// `part` (row length 9 * cin * cout + cout, bias partials at the end from the
-// tap-4 blocks); k_wgrad_sum then adds the rows up in slice order, so the
-// gradients, and the training built on them, are the same on every run.
+// Weight gradient: dW[tap][ci][co] = sum_p dpre[p][co] * in[p + off(tap)][ci],
+// db[co] = sum_p dpre[p][co]: a product with M = co, N = (tap, ci) and the
+// pixels as K. MFMA wants eight K values of one channel in a lane, while the
+// tensors are NHWC, so a tile of pixels is transposed on its way into LDS:
+// a thread loads eight channels of eight pixels (16 bytes each) and writes
+// eight 16-byte octets, one channel's eight pixels each (32 v_perm_b32 for 64
+// values). The eight pixels of an octet lie `tw` apart in their row (a tile is
+// 8 * tw pixels wide), not side by side: the octet of the neighbouring pixels
+// is then the neighbouring 16 bytes, so every tap's shifted operand is one
+// aligned 16-byte read, and the input is staged once for all nine taps, with a
+// one-pixel halo. Channels lie an odd number of octets apart, so the 16
+// channels that a read takes fall into different banks.
+//
+// A block owns a group of input channels, one 16-channel tile per wave, all
+// taps and all output channels (9 * MT accumulators a wave), and one slice of
+// the tiles; with few channel tiles `ksplit` waves share one and split its
+// K steps, adding up through LDS at the end. Slices store their sums to rows of
+// `part` (9 * cin * cout weights, then cout bias sums); k_wgrad_sum adds the
+// rows in slice order, so gradients, and the training built on them, are the
+// same on every run.
+//
+// What bounds it: the loads of the two tensors, once per channel group, and
+// their latency; the products alone take a few microseconds a layer. Over
+// eight 256 x 256 crops the fifteen layers take 0.40 ms; gathering each lane's
+// operands from untransposed LDS 16 bits at a time, and staging the input
+// once per tap, they took 7.8 ms (the training step 10.05 -> 2.40 ms).
 // ---------------------------------------------------------------------------
-constexpr int WG_MAX_PAIRS = 12;
-constexpr int WG_SLICES = 64;
+constexpr int WG_MAX_THREADS = 512;
+constexpr size_t WG_LDS = 160 * 1024;  // LDS of a CU
+constexpr int WG_CUS = 256;
 
-__global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ in, int cin, const bf16* __restrict__ dpre,
-                                               int cout, int n, int h, int w, int slices,
-                                               float* __restrict__ part) {
-    extern __shared__ unsigned char smem_raw[];
-    bf16* s_in = reinterpret_cast<bf16*>(smem_raw);  // [32][cin]
-    bf16* s_dp = s_in + 32 * cin;                    // [32][cout]
-    const int tap = blockIdx.x / slices, slice = blockIdx.x % slices;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int g = lane >> 4, r = lane & 15;
-    const int mts = cout / 16, nts = cin / 16;
-    const int pairs = mts * nts;
-    f32x4 acc[WG_MAX_PAIRS];
-#pragma unroll
-    for (int q = 0; q < WG_MAX_PAIRS; ++q) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float bsum = 0.0f;  // bias partial for channel threadIdx.x (tap 4 only)
-    const size_t pixels = (size_t)n * h * w;
-    const int chunks = (int)((pixels + 31) / 32);
-    const int per = (chunks + slices - 1) / slices;
-    const int c0 = slice * per, c1 = min(chunks, c0 + per);
-    for (int ch = c0; ch < c1; ++ch) {
-        const size_t p0 = (size_t)ch * 32;
-        __syncthreads();
-        // Stage: 32 pixels x cin of the shifted input, 32 x cout of dpre (16 B per load).
-        for (int e = threadIdx.x; e < 32 * cin / 8; e += 256) {
-            const int p = e / (cin / 8), part = e % (cin / 8);
-            const size_t pf = p0 + p;
-            const int x = (int)(pf % w), y = (int)((pf / w) % h);
-            const size_t img = pf / ((size_t)w * h);
-            const int sy = y + dy, sx = x + dx;
-            bf16x8 v;
-            if (pf < pixels && sy >= 0 && sy < h && sx >= 0 && sx < w) {
-                v = *reinterpret_cast<const bf16x8*>(in + ((img * h + sy) * w + sx) * cin + part * 8);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = f2b(0.0f);
-            }
-            *reinterpret_cast<bf16x8*>(s_in + p * cin + part * 8) = v;
-        }
-        for (int e = threadIdx.x; e < 32 * cout / 8; e += 256) {
-            const int p = e / (cout / 8), part = e % (cout / 8);
-            bf16x8 v;
-            if (p0 + p < pixels) {
-                v = *reinterpret_cast<const bf16x8*>(dpre + (p0 + p) * cout + part * 8);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = f2b(0.0f);
-            }
-            *reinterpret_cast<bf16x8*>(s_dp + p * cout + part * 8) = v;
-        }
-        __syncthreads();
-        if (tap == 4 && (int)threadIdx.x < cout)
-            for (int p = 0; p < 32; ++p) bsum += b2f(s_dp[p * cout + threadIdx.x]);
-        // K = the chunk's 32 pixels; lane's k-range is pixels 8g .. 8g+7.
-#pragma unroll
-        for (int q = 0; q < WG_MAX_PAIRS; ++q) {
-            const int pr = wv + 4 * q;
-            if (pr < pairs) {
-                const int mt = pr % mts, nt = pr / mts;
-                bf16x8 av, bv;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    av[i] = s_dp[(8 * g + i) * cout + mt * 16 + r];
-                    bv[i] = s_in[(8 * g + i) * cin + nt * 16 + r];
-                }
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[q], 0, 0, 0);
-            }
-        }
-    }
-    // D[m = co][n = ci]: lane holds co = mt*16 + 4g + j, ci = nt*16 + r.
-    float* row = part + (size_t)slice * ((size_t)9 * cin * cout + cout);
-#pragma unroll
-    for (int q = 0; q < WG_MAX_PAIRS; ++q) {
-        const int pr = wv + 4 * q;
-        if (pr < pairs) {
-            const int mt = pr % mts, nt = pr / mts;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int co = mt * 16 + 4 * g + j, ci = nt * 16 + r;
-                row[(tap * cin + ci) * cout + co] = acc[q][j];
-            }
-        }
-    }
-    if (tap == 4 && (int)threadIdx.x < cout) row[(size_t)9 * cin * cout + threadIdx.x] = bsum;
+struct WgradPlan {
+    int tw, rows;         // tile: 8 * tw pixels x rows
+    int nw, groups;       // channel tiles (waves) per group, groups
+    int ksplit, slices;   // waves per channel tile; slices of the tiles
+    int tiles_x, tiles_y, tiles;
+    int in_stride, dp_stride;  // octets from one channel to the next
+    size_t lds;
+};
+
+// Eight pixels (16 bytes of channels each) into eight octets (one channel each).
+__device__ inline void transpose8(const uint4 (&v)[8], uint4 (&o)[8]) {
+    const uint32_t lo = 0x05040100u, hi = 0x07060302u;  // the low, the high halves of two words
+#define LUCIDA_PAIR(c, m, sel)                                                              \
+    o[c] = make_uint4(__builtin_amdgcn_perm(v[1].m, v[0].m, sel), __builtin_amdgcn_perm(v[3].m, v[2].m, sel), \
+                      __builtin_amdgcn_perm(v[5].m, v[4].m, sel), __builtin_amdgcn_perm(v[7].m, v[6].m, sel))
+    LUCIDA_PAIR(0, x, lo);
+    LUCIDA_PAIR(1, x, hi);
+    LUCIDA_PAIR(2, y, lo);
+    LUCIDA_PAIR(3, y, hi);
+    LUCIDA_PAIR(4, z, lo);
+    LUCIDA_PAIR(5, z, hi);
+    LUCIDA_PAIR(6, w, lo);
+    LUCIDA_PAIR(7, w, hi);
+#undef LUCIDA_PAIR
 }
 
-// grad[e] = sum over slices k = 0, 1, ... of part[k][e], in that order.
-__global__ __launch_bounds__(256) void k_wgrad_sum(const float* __restrict__ part, size_t row, int slices,
+// Loads the octets' pixels of image row y, x = x0 + 8 values tw apart, eight
+// channels from c0; zeros outside the image.
+__device__ inline void load_octets(const bf16* __restrict__ t, int c, int c0, int img, int h, int w, int y, int x0,
+                                   int tw, uint4 (&v)[8]) {
+    const bool row = y >= 0 && y < h;
+    const bf16* base = t + ((size_t)img * h + (row ? y : 0)) * w * c + c0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int x = x0 + j * tw;
+        v[j] = make_uint4(0u, 0u, 0u, 0u);
+        if (row && x >= 0 && x < w) v[j] = *reinterpret_cast<const uint4*>(base + (size_t)x * c);
+    }
+}
+
+template <int MT>
+__global__ __launch_bounds__(MT > 4 ? 256 : WG_MAX_THREADS) void k_wgrad(const bf16* __restrict__ in, int cin,
+                                                          const bf16* __restrict__ dpre, int n, int h, int w,
+                                                          WgradPlan pl, float* __restrict__ part) {
+    extern __shared__ uint4 wg_lds[];
+    constexpr int cout = MT * 16;
+    const int tw = pl.tw, hw = tw + 2;
+    const int pos_in = (pl.rows + 2) * hw, pos_dp = pl.rows * tw;
+    uint4* s_in = wg_lds;                                    // [16 * nw][in_stride]
+    uint4* s_dp = wg_lds + (size_t)16 * pl.nw * pl.in_stride;  // [cout][dp_stride]
+    const int slice = blockIdx.x / pl.groups, group = blockIdx.x % pl.groups;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int ct = wv % pl.nw, ks = wv / pl.nw;  // channel tile in the group; share of its K steps
+    const int g = lane >> 4, r = lane & 15;
+    const bool bias_wave = group == 0 && ct == 0;
+    f32x4 acc[9][MT], accb[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        accb[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc[t][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ones[i] = f2b(1.0f);
+    const int oct_in = 2 * pl.nw;  // channel octets of the group
+    const int items_in = oct_in * pos_in, items = items_in + (cout / 8) * pos_dp;
+    for (int tile = slice; tile < pl.tiles; tile += pl.slices) {
+        const int tx = tile % pl.tiles_x, rest = tile / pl.tiles_x;
+        const int y0 = (rest % pl.tiles_y) * pl.rows, img = rest / pl.tiles_y;
+        const int x0 = tx * 8 * tw;
+        __syncthreads();  // the previous tile's reads are done
+        for (int e = threadIdx.x; e < items; e += blockDim.x) {
+            uint4 v[8], o[8];
+            uint4* dst;
+            int stride;
+            if (e < items_in) {
+                const int c8 = e % oct_in, p = e / oct_in;
+                load_octets(in, cin, group * pl.nw * 16 + 8 * c8, img, h, w, y0 + p / hw - 1, x0 + p % hw - 1, tw, v);
+                stride = pl.in_stride;
+                dst = s_in + (size_t)(8 * c8) * stride + p;
+            } else {
+                const int f = e - items_in, c8 = f % (cout / 8), p = f / (cout / 8);
+                load_octets(dpre, cout, 8 * c8, img, h, w, y0 + p / tw, x0 + p % tw, tw, v);
+                stride = pl.dp_stride;
+                dst = s_dp + (size_t)(8 * c8) * stride + p;
+            }
+            transpose8(v, o);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) dst[k * stride] = o[k];
+        }
+        __syncthreads();
+        // K steps of 32 pixels: lane group g takes position 4s + g
+        for (int s = ks; s < pos_dp / 4; s += pl.ksplit) {
+            const int p = 4 * s + g;
+            const uint4* a = s_dp + (size_t)r * pl.dp_stride + p;
+            const uint4* b = s_in + (size_t)(ct * 16 + r) * pl.in_stride + (p / tw) * hw + p % tw;
+            bf16x8 av[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) av[m] = *reinterpret_cast<const bf16x8*>(a + (size_t)m * 16 * pl.dp_stride);
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const bf16x8 bv = *reinterpret_cast<const bf16x8*>(b + (t / 3) * hw + t % 3);
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv, acc[t][m], 0, 0, 0);
+            }
+            if (bias_wave) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], ones, accb[m], 0, 0, 0);
+            }
+        }
+    }
+    // The K shares of a channel tile, added up in order by the first, one
+    // output tile at a time (so the staging space is enough).
+    f32x4* s_red = reinterpret_cast<f32x4*>(wg_lds) + (size_t)ct * 10 * 64 + lane;
+    for (int k = 1; k < pl.ksplit; ++k) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            __syncthreads();
+            if (ks == k) {
+                s_red[9 * 64] = accb[m];
+#pragma unroll
+                for (int t = 0; t < 9; ++t) s_red[t * 64] = acc[t][m];
+            }
+            __syncthreads();
+            if (ks == 0) {
+                accb[m] += s_red[9 * 64];
+#pragma unroll
+                for (int t = 0; t < 9; ++t) acc[t][m] += s_red[t * 64];
+            }
+        }
+    }
+    if (ks != 0) return;
+    // D[m = co][n = ci]: lane holds co = m*16 + 4g + j, ci = the tile's r.
+    float* row = part + (size_t)slice * ((size_t)9 * cin * cout + cout);
+    const int ci = (group * pl.nw + ct) * 16 + r;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            *reinterpret_cast<f32x4*>(row + ((size_t)t * cin + ci) * cout + m * 16 + 4 * g) = acc[t][m];
+    if (bias_wave && r == 0) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            *reinterpret_cast<f32x4*>(row + (size_t)9 * cin * cout + m * 16 + 4 * g) = accb[m];
+    }
+}
+
+// grad[e] = the sum of part[k][e] over the slices: four threads an element,
+// each every fourth slice in ascending order, then the four in order. With one
+// thread an element the small layers' few blocks waited for one load after
+// another.
+__global__ __launch_bounds__(256) void k_wgrad_sum(const float* __restrict__ part, uint32_t row, int slices,
                                                    float* __restrict__ grad) {
-    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= row) return;
+    __shared__ float red[256];
+    const uint32_t e = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int q = threadIdx.x >> 6;
     float acc = 0.0f;
-    for (int k = 0; k < slices; ++k) acc += part[(size_t)k * row + e];
-    grad[e] = acc;
+    if (e < row) {
+#pragma unroll 8
+        for (int k = q; k < slices; k += 4) acc += part[(size_t)k * row + e];
+    }
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    if (q == 0 && e < row) grad[e] = ((red[threadIdx.x] + red[threadIdx.x + 64]) + red[threadIdx.x + 128]) + red[threadIdx.x + 192];
 }
 
 // ---------------------------------------------------------------------------
@@ -495,6 +586,9 @@ const NetLayer kNetLayers[kNetNumLayers] = {
     {160, 64, 1}, {64, 64, 1},  {112, 48, 1}, {48, 48, 1}, {80, 32, 1}, {32, 32, 1}, {32, 16, 0},
 };
 
+// Resolution level of each layer (level k is 2^k smaller per side).
+static const int kNetLevel[kNetNumLayers] = {0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 1, 1, 0, 0, 0};
+
 size_t net_param_count() {
     size_t c = 0;
     for (const auto& l : kNetLayers) c += (size_t)9 * l.cin * l.cout + l.cout;
@@ -540,6 +634,58 @@ static lucida_status launch_conv(hipStream_t s, const bf16* in, int cin, int cou
     return LUCIDA_OK;
 }
 
+// How a layer's weight gradient is split. Tiles are 64 pixels wide where the
+// row allows, else 32 or 16 (rows are multiples of 16). A wave holds 9 * MT
+// accumulators of 4 registers, so a block of up to eight waves (256 registers
+// each) serves MT up to 4 and one of four waves MT = 6. Few channel tiles
+// (16 or 32 channels) share the K steps of larger tiles among more waves.
+// Slices: as many blocks as the CUs hold at once (one or two each, by LDS), as
+// every slice costs a row of partial sums written and read.
+static WgradPlan plan_wgrad(int cin, int cout, int n, int h, int w) {
+    WgradPlan p{};
+    const int ct = cin / 16, mt = cout / 16;
+    const int max_waves = mt > 4 ? 4 : WG_MAX_THREADS / 64;
+    p.groups = 1;
+    while (ct % p.groups != 0 || ct / p.groups > max_waves) ++p.groups;
+    p.nw = ct / p.groups;
+    p.ksplit = 1;
+    while (p.nw * p.ksplit * 2 <= max_waves) p.ksplit *= 2;
+    const int pos = p.ksplit >= 4 ? 64 : 32;  // octets of 8 pixels per tile
+    p.tw = w % 64 == 0 ? 8 : (w % 32 == 0 ? 4 : 2);
+    p.rows = pos / p.tw;
+    p.tiles_x = w / (8 * p.tw);
+    p.tiles_y = (h + p.rows - 1) / p.rows;
+    p.tiles = n * p.tiles_x * p.tiles_y;
+    p.in_stride = ((p.rows + 2) * (p.tw + 2)) | 1;
+    p.dp_stride = (p.rows * p.tw) | 1;
+    p.lds = (size_t)16 * (16 * p.nw * p.in_stride + cout * p.dp_stride);
+    if (p.ksplit > 1) p.lds = std::max(p.lds, (size_t)p.nw * 10 * 1024);
+    const int resident = p.lds > WG_LDS / 2 ? 1 : 2;  // blocks a CU
+    p.slices = std::max(1, std::min(p.tiles, resident * WG_CUS / p.groups));
+    return p;
+}
+
+template <int MT>
+static lucida_status launch_wgrad_t(hipStream_t s, const bf16* in, int cin, const bf16* dpre, int n, int h, int w,
+                                    const WgradPlan& p, float* part) {
+    if (p.lds > WG_LDS) return set_error(LUCIDA_INVALID_ARG, "weight gradient: tile larger than LDS");
+    hipLaunchKernelGGL((k_wgrad<MT>), dim3(p.slices * p.groups), dim3(64 * p.nw * p.ksplit), p.lds, s, in, cin, dpre,
+                       n, h, w, p, part);
+    return LUCIDA_OK;
+}
+
+static lucida_status launch_wgrad(hipStream_t s, const bf16* in, int cin, const bf16* dpre, int cout, int n, int h,
+                                  int w, const WgradPlan& p, float* part) {
+    switch (cout / 16) {
+        case 1: return launch_wgrad_t<1>(s, in, cin, dpre, n, h, w, p, part);
+        case 2: return launch_wgrad_t<2>(s, in, cin, dpre, n, h, w, p, part);
+        case 3: return launch_wgrad_t<3>(s, in, cin, dpre, n, h, w, p, part);
+        case 4: return launch_wgrad_t<4>(s, in, cin, dpre, n, h, w, p, part);
+        case 6: return launch_wgrad_t<6>(s, in, cin, dpre, n, h, w, p, part);
+        default: return set_error(LUCIDA_INVALID_ARG, "weight gradient: unsupported output channel count");
+    }
+}
+
 static size_t frag_elems(int in_c, int out_c) {
     const int kbs = 9 * in_c / 16;
     return (size_t)((kbs + 1) / 2) * (out_c / 16) * 64 * 8;
@@ -554,7 +700,7 @@ using namespace lucida;
 struct lucida_net {
     lucida_ctx* ctx = nullptr;
     DevBuf params, grads, adam_m, adam_v;  // fp32, layout: per layer W[9][cin][cout] then b[cout]
-    DevBuf wg_part;                        // weight-gradient partials: WG_SLICES rows of one layer's W and b
+    DevBuf wg_part;                        // weight-gradient partials: a row of one layer's W and b per slice
     DevBuf frag_fwd, frag_bwd;             // bf16 fragments
     size_t frag_fwd_off[kNetNumLayers], frag_bwd_off[kNetNumLayers], param_off[kNetNumLayers];
     DevBuf acts, dacts, target, loss_partial;
@@ -588,8 +734,7 @@ static ActPlan plan_acts(int n, int h, int w) {
     };
     const int H[4] = {h, h / 2, h / 4, h / 8}, Wd[4] = {w, w / 2, w / 4, w / 8};
     a.x = take(H[0], Wd[0], 16);
-    const int lvl[15] = {0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 1, 1, 0, 0, 0};
-    for (int i = 0; i < 15; ++i) a.l[i] = take(H[lvl[i]], Wd[lvl[i]], kNetLayers[i].cout);
+    for (int i = 0; i < 15; ++i) a.l[i] = take(H[kNetLevel[i]], Wd[kNetLevel[i]], kNetLayers[i].cout);
     a.p0 = take(H[1], Wd[1], 32);
     a.p1 = take(H[2], Wd[2], 48);
     a.p2 = take(H[3], Wd[3], 64);
@@ -704,11 +849,18 @@ static lucida_status net_backward(lucida_net* net) {
     const bf16* FB = net->frag_bwd.as<bf16>();
     const int H[4] = {H0, H0 / 2, H0 / 4, H0 / 8}, Wd[4] = {W0, W0 / 2, W0 / 4, W0 / 8};
     // Every layer's W and b gradients are written whole by its k_wgrad_sum;
-    // the partials buffer is sized once, for the largest layer.
-    size_t max_row = 0;
-    for (int li = 0; li < kNetNumLayers; ++li)
-        max_row = std::max(max_row, (size_t)9 * kNetLayers[li].cin * kNetLayers[li].cout + kNetLayers[li].cout);
-    LUCIDA_HIP(net->wg_part.ensure((size_t)WG_SLICES * max_row * 4), LUCIDA_OOM);
+    // the partials buffer is sized for the layer with the most.
+    WgradPlan wg[kNetNumLayers];
+    size_t max_part = 0;
+    for (int li = 0; li < kNetNumLayers; ++li) {
+        const NetLayer& L = kNetLayers[li];
+        wg[li] = plan_wgrad(L.cin, L.cout, n, H[kNetLevel[li]], Wd[kNetLevel[li]]);
+        max_part = std::max(max_part, (size_t)wg[li].slices * ((size_t)9 * L.cin * L.cout + L.cout));
+    }
+    if (max_part * 4 > net->wg_part.bytes) {
+        LUCIDA_HIP(hipStreamSynchronize(s), LUCIDA_VALIDATION);
+        LUCIDA_HIP(net->wg_part.ensure(max_part * 4), LUCIDA_OOM);
+    }
     lucida_status st;
     // d(layer li's pre-activation) -> weight grads, and d(its input) into d_in.
     auto layer_bwd = [&](int li, size_t in_off, int lvl, size_t d_in_off) -> lucida_status {
@@ -716,14 +868,12 @@ static lucida_status net_backward(lucida_net* net) {
         const size_t count = (size_t)n * H[lvl] * Wd[lvl] * L.cout;
         if (L.relu)
             hipLaunchKernelGGL(k_relu_bwd, dim3(grid1(count)), dim3(256), 0, s, D + a.l[li], A + a.l[li], count);
-        if ((L.cin / 16) * (L.cout / 16) > 4 * WG_MAX_PAIRS)
-            return set_error(LUCIDA_INVALID_ARG, "weight gradient: too many channel tiles for one block");
-        const size_t lds = (size_t)32 * (L.cin + L.cout) * 2;
-        const size_t row = (size_t)9 * L.cin * L.cout + L.cout;  // the layer's W then b, as in `grads`
-        hipLaunchKernelGGL(k_wgrad, dim3(9 * WG_SLICES), dim3(256), lds, s, A + in_off, L.cin, D + a.l[li], L.cout,
-                           n, H[lvl], Wd[lvl], WG_SLICES, net->wg_part.as<float>());
-        hipLaunchKernelGGL(k_wgrad_sum, dim3((unsigned)((row + 255) / 256)), dim3(256), 0, s,
-                           net->wg_part.as<float>(), row, WG_SLICES, G + net->param_off[li]);
+        const uint32_t row = (uint32_t)(9 * L.cin * L.cout + L.cout);  // the layer's W then b, as in `grads`
+        const lucida_status ws = launch_wgrad(s, A + in_off, L.cin, D + a.l[li], L.cout, n, H[lvl], Wd[lvl], wg[li],
+                                              net->wg_part.as<float>());
+        if (ws != LUCIDA_OK) return ws;
+        hipLaunchKernelGGL(k_wgrad_sum, dim3((row + 63) / 64), dim3(256), 0, s, net->wg_part.as<float>(), row,
+                           wg[li].slices, G + net->param_off[li]);
         if (d_in_off == (size_t)-1) return LUCIDA_OK;
         return launch_conv(s, D + a.l[li], L.cout, L.cin, FB + net->frag_bwd_off[li], nullptr, 0, D + d_in_off, n,
                            H[lvl], Wd[lvl]);
