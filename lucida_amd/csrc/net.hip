@@ -8,11 +8,13 @@
 // Convolutions are implicit GEMMs on v_mfma_f32_16x16x32_bf16 with the output
 // channels as the GEMM's M side: a wave computes 16 output channels x 16
 // consecutive pixels of one row per instruction, the K side walks (tap,
-// 16-channel block) pairs. Activations are NHWC BF16 so every lane loads its
-// 8 K-values with one 16-byte load; weights are pre-swizzled into per-lane
-// fragments so every wave reads them with one coalesced 1 KB load per tile.
-// The input-gradient pass is the same kernel over transposed, tap-flipped
-// weights; the weight-gradient pass transposes pixel tiles through LDS.
+// 16-channel block) pairs. Activations are NHWC BF16, staged in LDS by tile, so
+// every lane reads its 8 K-values with one 16-byte read; weights are
+// pre-swizzled into per-lane fragments so every wave reads them with one
+// coalesced 1 KB load per tile. Pooling, the concatenations and their
+// gradients happen inside the convolutions. The input-gradient pass is the same
+// kernel over transposed, tap-flipped weights; the weight-gradient pass
+// transposes pixel tiles through LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,11 +37,21 @@ __device__ inline float b2f(bf16 v) { return (float)v; }
 __device__ inline bf16 f2b(float v) { return (bf16)v; }
 
 // ---------------------------------------------------------------------------
+// Output channels of an MFMA tile's rows. Tiles go in pairs of 32 channels: row
+// 4g + j of the pair's tile q is channel 32 * pair + 8g + 4q + j, so the lane that
+// holds rows 4g .. 4g + 3 of both tiles holds eight consecutive channels (one
+// 16-byte store). The last tile of an odd count keeps its rows in order.
+// ---------------------------------------------------------------------------
+__device__ inline int tile_channel(int mt, int tiles, int row) {
+    return (mt | 1) < tiles ? 32 * (mt >> 1) + 8 * (row >> 2) + 4 * (mt & 1) + (row & 3) : 16 * mt + row;
+}
+
+// ---------------------------------------------------------------------------
 // Weight preparation: FP32 master weights W[tap][ci][co] -> BF16 fragments.
-// Fragment (chunk c, m-tile mt, lane l, i) holds A[co][k] with co = mt*16 +
-// l%16 and k = the i-th of 8 consecutive input channels of K-block
-// kb = 2c + (l/16)/2, half (l/16)%2. transpose = 1 builds the input-gradient
-// weights W'[tap][co][ci] = W[8 - tap][ci][co].
+// Fragment (chunk c, m-tile mt, lane l, i) holds A[co][k] with co =
+// tile_channel(mt, row l%16) and k = the i-th of 8 consecutive input channels of
+// K-block kb = 2c + (l/16)/2, half (l/16)%2. transpose = 1 builds the
+// input-gradient weights W'[tap][co][ci] = W[8 - tap][ci][co].
 // ---------------------------------------------------------------------------
 __global__ void k_wprep(const float* __restrict__ W, int cin, int cout, int transpose, bf16* __restrict__ frag) {
     const int in_c = transpose ? cout : cin;     // channels the fragment's K walks
@@ -57,7 +69,7 @@ __global__ void k_wprep(const float* __restrict__ W, int cin, int cout, int tran
         if (kb < kbs) {
             const int tap = kb / (in_c / 16), cb = kb % (in_c / 16);
             const int k_ch = cb * 16 + 8 * (g & 1) + i;  // input channel of the GEMM
-            const int m_ch = mt * 16 + r;                 // output channel of the GEMM
+            const int m_ch = tile_channel(mt, mts, r);    // output channel of the GEMM
             v = transpose ? W[((8 - tap) * cin + m_ch) * cout + k_ch] : W[(tap * cin + k_ch) * cout + m_ch];
         }
         frag[e] = f2b(v);
@@ -66,89 +78,294 @@ __global__ void k_wprep(const float* __restrict__ W, int cin, int cout, int tran
 
 // ---------------------------------------------------------------------------
 // Convolution (forward, or input gradient with prepared weights).
-// in:  NHWC bf16 [n][h][w][cin]; out: [n][h][w][MT*16]. One wave: NT tiles
-// of 16 consecutive pixels of a row (w % (16 * NT) == 0); each K chunk's
-// weight fragments are loaded once and used for all NT tiles, and every
-// output keeps the same sequence of MFMAs whatever NT is. bias (optional,
-// fp32) and ReLU fused in the epilogue.
+//
+// A block computes 32 pixels x `rows` rows of all output channels. It stages the
+// input tile, with its one-pixel halo and all input channels, in LDS (NHWC; the
+// 16-byte octets of a pixel and one pad octet, an odd number, so that the 16
+// pixels of a fragment read fall into different banks); its waves split the
+// rows (`wn`) and the output tiles (`wm`), and a wave keeps NT tiles of 16 pixels x
+// MTW tiles of 16 channels in registers. K walks (tap, 16-channel block) pairs as
+// the fragments do, so an output's sequence of MFMAs does not depend on the
+// split. Weight fragments come from L2, PF chunks ahead of their use.
+//
+// The input may be the concatenation of a half-resolution tensor (nearest 2x
+// upsampling, the first c_low channels) and a full-resolution one; it is then
+// read from the two directly and never written out. The epilogue (EPI) does
+// what would otherwise be passes of their own over the output:
+//   CONV_FWD        bias and ReLU
+//   CONV_FWD_POOL   the same, and the 2x2 average pool of the result to out2
+//   CONV_BWD        the ReLU mask of the layer below (its output `mask`)
+//   CONV_BWD_SPLIT  the gradient of the concatenation: the first c_split
+//                   channels summed over 2x2 and masked, the rest to out2
+//   CONV_BWD_UNPOOL the gradient through the pool: a quarter of the result
+//                   plus the skip branch's gradient `add` at each of the four
+//                   pixels, masked
+// Each rounds to BF16 where a separate pass would have read BF16, so results are
+// the same bit for bit.
+// What bounds it: staging and products share a block's time without overlapping
+// inside it, so it lives from the two or three blocks that a CU's LDS holds.
+// Inference of 1024 x 1024: the fifteen layers with their pools and
+// concatenations took 858 us with every wave reading its operands from L2 for
+// 32 pixels and the passes apart, 535 us so; the four passes of a training
+// step's backward (masks, pools, concatenations) took 400 us and are gone.
 // ---------------------------------------------------------------------------
-template <int MT, int NT>
-__global__ __launch_bounds__(256) void k_conv(const bf16* __restrict__ in, int cin, const bf16x8* __restrict__ frag,
-                                              const float* __restrict__ bias, int relu, bf16* __restrict__ out,
-                                              int n, int h, int w) {
-    const int lane = threadIdx.x & 63;
-    const int wave = (blockIdx.x * (blockDim.x >> 6)) + (threadIdx.x >> 6);
-    const int row_tiles = w / (16 * NT);
-    const int tiles = n * h * row_tiles;
-    if (wave >= tiles) return;
-    const int xt = wave % row_tiles, rowi = wave / row_tiles;
-    const int y = rowi % h, img = rowi / h;
-    const int x0 = xt * 16 * NT;
+enum { CONV_FWD, CONV_FWD_POOL, CONV_BWD, CONV_BWD_SPLIT, CONV_BWD_UNPOOL };
+constexpr int CONV_BW = 32;           // a block's pixels per row
+constexpr int CONV_LW = CONV_BW + 2;  // with the halo
+constexpr int CONV_STAGE = 10;        // loads in flight a thread while staging
+
+// An NHWC tensor of c_low + c channels: the first c_low from `low` at half the
+// resolution (c_low = 0: none).
+struct ConvSource {
+    const bf16* low;
+    const bf16* src;
+    int c_low, c;
+};
+
+struct ConvArgs {
+    ConvSource in;
+    const bf16x8* frag;
+    const float* bias;
+    bf16* out;
+    bf16* out2;
+    const bf16* mask;
+    const bf16* add;
+    int n, h, w;
+    int mts;               // output tiles of 16 channels
+    int relu, c_split;
+    int wm, wn, rows;      // waves along channels and rows; rows per block
+    int tiles_x, tiles_y;
+};
+
+// Blocks go to the eight XCDs in turn; block b of n works on a tile such that
+// each XCD's blocks cover one run of tiles, whose halos then meet in its L2.
+__device__ inline int xcd_order(uint32_t b, uint32_t n) {
+    const uint32_t per = n / 8, rem = n % 8, x = b % 8;
+    return (int)(x * per + min(x, rem) + b / 8);
+}
+
+// The value of lane ^ 1 (DPP quad_perm [1, 0, 3, 2]).
+__device__ inline float swap_pair(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
+}
+
+// V consecutive channels from ch of the wave's pixels: acc[t][0 .. V) of its
+// NT tiles (row t / 2, columns 16 * (t % 2) + r).
+template <int EPI, int NT, int V, class Acc>
+__device__ inline void conv_emit(const ConvArgs& a, int img, int y0, int x0, int r, int ch, Acc acc) {
+    typedef __bf16 vec __attribute__((ext_vector_type(V)));
+    const int cout = a.mts * 16;
+    float bias[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) bias[i] = a.bias ? a.bias[ch + i] : 0.0f;
+#pragma unroll
+    for (int rp = 0; rp < NT / 4; ++rp)
+#pragma unroll
+        for (int xt = 0; xt < 2; ++xt) {
+            const int x = x0 + 16 * xt + r, y = y0 + 2 * rp;
+            if (x >= a.w) continue;  // whole tiles: widths are multiples of 16
+            vec v[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    float s = acc(2 * (2 * rp + k) + xt, i) + bias[i];
+                    if ((EPI == CONV_FWD || EPI == CONV_FWD_POOL) && a.relu) s = fmaxf(s, 0.0f);
+                    v[k][i] = f2b(s);
+                }
+            if (EPI == CONV_FWD || EPI == CONV_FWD_POOL || EPI == CONV_BWD) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    if (y + k >= a.h) continue;
+                    const size_t at = (((size_t)img * a.h + y + k) * a.w + x) * cout + ch;
+                    if (EPI == CONV_BWD) {
+                        const vec m = *reinterpret_cast<const vec*>(a.mask + at);
+#pragma unroll
+                        for (int i = 0; i < V; ++i)
+                            if (!(b2f(m[i]) > 0.0f)) v[k][i] = f2b(0.0f);
+                    }
+                    *reinterpret_cast<vec*>(a.out + at) = v[k];
+                }
+            }
+            if (EPI == CONV_FWD_POOL || (EPI == CONV_BWD_SPLIT && ch < a.c_split)) {
+                // the 2x2 block of an even lane and its neighbour, summed
+                // left to right, top to bottom (pooled sizes are whole)
+                float s[V];
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const float p = b2f(v[0][i]), q = b2f(v[1][i]);
+                    s[i] = p + swap_pair(p) + q + swap_pair(q);
+                }
+                if (!(r & 1) && y < a.h) {
+                    const int c2 = EPI == CONV_FWD_POOL ? cout : a.c_split;
+                    const size_t at = (((size_t)img * (a.h / 2) + y / 2) * (a.w / 2) + x / 2) * c2 + ch;
+                    vec o;
+                    if (EPI == CONV_FWD_POOL) {
+#pragma unroll
+                        for (int i = 0; i < V; ++i) o[i] = f2b(0.25f * s[i]);
+                        *reinterpret_cast<vec*>(a.out2 + at) = o;
+                    } else {
+                        const vec m = *reinterpret_cast<const vec*>(a.mask + at);
+#pragma unroll
+                        for (int i = 0; i < V; ++i) o[i] = f2b(b2f(m[i]) > 0.0f ? s[i] : 0.0f);
+                        *reinterpret_cast<vec*>(a.out + at) = o;
+                    }
+                }
+            }
+            if (EPI == CONV_BWD_SPLIT && ch >= a.c_split) {
+                const int c2 = cout - a.c_split;
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    if (y + k < a.h)
+                        *reinterpret_cast<vec*>(a.out2 + (((size_t)img * a.h + y + k) * a.w + x) * c2 + ch -
+                                                a.c_split) = v[k];
+            }
+            if (EPI == CONV_BWD_UNPOOL) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    if (y + k >= a.h) continue;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const size_t at = (((size_t)img * 2 * a.h + 2 * (y + k) + q / 2) * 2 * a.w + 2 * x + q % 2) * cout + ch;
+                        const vec d = *reinterpret_cast<const vec*>(a.add + at);
+                        const vec m = *reinterpret_cast<const vec*>(a.mask + at);
+                        vec o;
+#pragma unroll
+                        for (int i = 0; i < V; ++i)
+                            o[i] = f2b(b2f(m[i]) > 0.0f ? 0.25f * b2f(v[k][i]) + b2f(d[i]) : 0.0f);
+                        *reinterpret_cast<vec*>(a.out + at) = o;
+                    }
+                }
+            }
+        }
+}
+
+template <int MTW, int NT, int PF, int EPI>
+__global__ __launch_bounds__(512) void k_conv(ConvArgs a) {
+    extern __shared__ uint4 cv_lds[];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int wmi = wv % a.wm, wni = wv / a.wm;
     const int g = lane >> 4, r = lane & 15;
-    const int cbs = cin / 16;
-    const int kbs = 9 * cbs;
-    const int chunks = (kbs + 1) / 2;
-    f32x4 acc[NT][MT];
+    const int tile = xcd_order(blockIdx.x, gridDim.x);
+    const int tx = tile % a.tiles_x, rest = tile / a.tiles_x;
+    const int by = (rest % a.tiles_y) * a.rows, img = rest / a.tiles_y;
+    const int x0 = tx * CONV_BW;
+    const int cin = a.in.c_low + a.in.c;
+    const int octs = cin / 8, S = octs + 1;
+    // Stage: consecutive threads take consecutive octets of the tile's pixels,
+    // CONV_STAGE loads in flight a thread.
+    {
+        const bf16* lowi = a.in.low + (size_t)img * (a.h / 2) * (a.w / 2) * a.in.c_low;
+        const bf16* srci = a.in.src + (size_t)img * a.h * a.w * a.in.c;
+        const int step_o = blockDim.x % octs, step_p = blockDim.x / octs;
+        int o = threadIdx.x % octs, p = threadIdx.x / octs;
+        int ry = p / CONV_LW, px = p - ry * CONV_LW;
+        while (ry < a.rows + 2) {
+            uint4 v[CONV_STAGE];
+            int at[CONV_STAGE];
+#pragma unroll
+            for (int k = 0; k < CONV_STAGE; ++k) {
+                const int x = x0 - 1 + px, y = by - 1 + ry;
+                at[k] = ry < a.rows + 2 ? (ry * CONV_LW + px) * S + o : -1;
+                v[k] = make_uint4(0u, 0u, 0u, 0u);
+                if (at[k] >= 0 && x >= 0 && x < a.w && y >= 0 && y < a.h) {
+                    const bool low = 8 * o < a.in.c_low;
+                    const uint32_t i = low ? ((uint32_t)(y >> 1) * (a.w / 2) + (x >> 1)) * a.in.c_low + 8 * o
+                                           : ((uint32_t)y * a.w + x) * a.in.c + 8 * o - a.in.c_low;
+                    v[k] = *reinterpret_cast<const uint4*>((low ? lowi : srci) + i);
+                }
+                o += step_o;
+                px += step_p;
+                if (o >= octs) {
+                    o -= octs;
+                    ++px;
+                }
+                while (px >= CONV_LW) {
+                    px -= CONV_LW;
+                    ++ry;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < CONV_STAGE; ++k)
+                if (at[k] >= 0) cv_lds[at[k]] = v[k];
+        }
+    }
+    const int cbs = cin / 16, kbs = 9 * cbs, chunks = (kbs + 1) / 2;
+    const int mt0 = wmi * MTW;
+    const bf16x8* fp[MTW];  // the wave's fragments of a chunk (a tile past the last repeats it)
+#pragma unroll
+    for (int m = 0; m < MTW; ++m) fp[m] = a.frag + (size_t)min(mt0 + m, a.mts - 1) * 64 + lane;
+    const size_t fstep = (size_t)a.mts * 64;
+    bf16x8 av[PF][MTW];
+#pragma unroll
+    for (int i = 0; i < PF; ++i)
+#pragma unroll
+        for (int m = 0; m < MTW; ++m) av[i][m] = fp[m][fstep * min(i, chunks - 1)];
+    f32x4 acc[NT][MTW];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // A chunk's weight fragments and input columns; chunk c + 1's loads are
-    // issued before chunk c's products, so a wave keeps its next loads in
-    // flight while its MFMAs run.
-    auto load_chunk = [&](int c, bf16x8* av, bf16x8* bv) {
-        const int kb = 2 * c + (g >> 1);
-        const bool kok = kb < kbs;
-        int tap = 0, cb = 0;
-        if (kok) {
-            tap = kb / cbs;
-            cb = kb - tap * cbs;
-        }
-        const int sy = y + tap / 3 - 1;
-        const bool yok = kok && sy >= 0 && sy < h;
+        for (int m = 0; m < MTW; ++m) acc[t][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int wrow = wni * (NT / 2);  // the wave's first row in the tile
+    const uint4* bp = cv_lds + (size_t)(wrow * CONV_LW + r) * S + (g & 1);
+    int tap0 = 0, cb0 = 0;  // of the chunk's first K-block
+    __syncthreads();
+    for (int c0 = 0; c0 < chunks; c0 += PF) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m) av[m] = frag[(c * MT + m) * 64 + lane];
+        for (int i = 0; i < PF; ++i) {
+            const int c = c0 + i;
+            if (c < chunks) {
+                // the chunk's two K-blocks; an odd count's missing last one has
+                // zero weights and reads zeros
+                int tap1 = tap0, cb1 = cb0 + 1;
+                if (cb1 == cbs) {
+                    cb1 = 0;
+                    ++tap1;
+                }
+                const bool pad = tap1 == 9;
+                const int off0 = (tap0 / 3 * CONV_LW + tap0 % 3) * S + 2 * cb0;
+                const int off1 = pad ? off0 : (tap1 / 3 * CONV_LW + tap1 % 3) * S + 2 * cb1;
+                const uint4* q = bp + (g < 2 ? off0 : off1);
+                uint4 bv[NT];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int sx = x0 + 16 * t + r + tap % 3 - 1;
-            if (yok && sx >= 0 && sx < w) {
-                bv[t] = *reinterpret_cast<const bf16x8*>(in + (((size_t)img * h + sy) * w + sx) * cin + cb * 16 +
-                                                         8 * (g & 1));
-            } else {
+                for (int t = 0; t < NT; ++t) bv[t] = q[((t / 2) * CONV_LW + 16 * (t % 2)) * S];
+                if (pad && g >= 2) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) bv[t][i] = f2b(0.0f);
+                    for (int t = 0; t < NT; ++t) bv[t] = make_uint4(0u, 0u, 0u, 0u);
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int m = 0; m < MTW; ++m)
+                        acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i][m], __builtin_bit_cast(bf16x8, bv[t]),
+                                                                            acc[t][m], 0, 0, 0);
+                cb0 = cb1 + 1;
+                tap0 = tap1;
+                if (cb0 == cbs) {
+                    cb0 = 0;
+                    ++tap0;
+                }
+                const int cn = c + PF;
+                if (cn < chunks) {
+#pragma unroll
+                    for (int m = 0; m < MTW; ++m) av[i][m] = fp[m][fstep * cn];
+                }
             }
         }
-    };
-    bf16x8 av[MT], bv[NT], av_next[MT], bv_next[NT];
-    load_chunk(0, av_next, bv_next);
-    for (int c = 0; c < chunks; ++c) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m) av[m] = av_next[m];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) bv[t] = bv_next[t];
-        if (c + 1 < chunks) load_chunk(c + 1, av_next, bv_next);
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv[t], acc[t][m], 0, 0, 0);
     }
-    const int cout = MT * 16;
+    // D: lane holds rows 4g + j of each output tile, pixel column r.
+    const int y = by + wrow;
+    if (y >= a.h) return;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        bf16* o = out + (((size_t)img * h + y) * w + x0 + 16 * t + r) * cout;
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            bf16x4 v;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int co = m * 16 + 4 * g + j;
-                float s = acc[t][m][j] + (bias ? bias[co] : 0.0f);
-                if (relu) s = fmaxf(s, 0.0f);
-                v[j] = f2b(s);
-            }
-            *reinterpret_cast<bf16x4*>(o + m * 16 + 4 * g) = v;
+    for (int m = 0; m < MTW; m += 2) {
+        const int mt = mt0 + m;
+        if (mt >= a.mts) continue;
+        if (m + 1 < MTW && mt + 1 < a.mts) {  // a pair (mt0 is even then)
+            conv_emit<EPI, NT, 8>(a, img, y, x0, r, 16 * mt + 8 * g,
+                                  [&](int t, int i) { return i < 4 ? acc[t][m][i] : acc[t][m + 1 < MTW ? m + 1 : m][i - 4]; });
+        } else {
+            conv_emit<EPI, NT, 4>(a, img, y, x0, r, tile_channel(mt, a.mts, 4 * g),
+                                  [&](int t, int i) { return acc[t][m][i]; });
         }
     }
 }
@@ -212,25 +429,28 @@ __device__ inline void transpose8(const uint4 (&v)[8], uint4 (&o)[8]) {
 }
 
 // Loads the octets' pixels of image row y, x = x0 + 8 values tw apart, eight
-// channels from c0; zeros outside the image.
-__device__ inline void load_octets(const bf16* __restrict__ t, int c, int c0, int img, int h, int w, int y, int x0,
-                                   int tw, uint4 (&v)[8]) {
+// channels from c0 (a multiple of 8); zeros outside the image.
+__device__ inline void load_octets(const ConvSource& t, int c0, int img, int h, int w, int y, int x0, int tw,
+                                   uint4 (&v)[8]) {
     const bool row = y >= 0 && y < h;
-    const bf16* base = t + ((size_t)img * h + (row ? y : 0)) * w * c + c0;
+    const bool low = c0 < t.c_low;
+    const int sh = low ? 1 : 0, c = low ? t.c_low : t.c;
+    const bf16* base = (low ? t.low + c0 : t.src + (c0 - t.c_low)) +
+                       ((size_t)img * (h >> sh) + ((row ? y : 0) >> sh)) * (w >> sh) * c;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int x = x0 + j * tw;
         v[j] = make_uint4(0u, 0u, 0u, 0u);
-        if (row && x >= 0 && x < w) v[j] = *reinterpret_cast<const uint4*>(base + (size_t)x * c);
+        if (row && x >= 0 && x < w) v[j] = *reinterpret_cast<const uint4*>(base + (size_t)(x >> sh) * c);
     }
 }
 
 template <int MT>
-__global__ __launch_bounds__(MT > 4 ? 256 : WG_MAX_THREADS) void k_wgrad(const bf16* __restrict__ in, int cin,
-                                                          const bf16* __restrict__ dpre, int n, int h, int w,
+__global__ __launch_bounds__(MT > 4 ? 256 : WG_MAX_THREADS) void k_wgrad(ConvSource in, ConvSource dpre, int h, int w,
                                                           WgradPlan pl, float* __restrict__ part) {
     extern __shared__ uint4 wg_lds[];
     constexpr int cout = MT * 16;
+    const int cin = in.c_low + in.c;
     const int tw = pl.tw, hw = tw + 2;
     const int pos_in = (pl.rows + 2) * hw, pos_dp = pl.rows * tw;
     uint4* s_in = wg_lds;                                    // [16 * nw][in_stride]
@@ -263,12 +483,12 @@ __global__ __launch_bounds__(MT > 4 ? 256 : WG_MAX_THREADS) void k_wgrad(const b
             int stride;
             if (e < items_in) {
                 const int c8 = e % oct_in, p = e / oct_in;
-                load_octets(in, cin, group * pl.nw * 16 + 8 * c8, img, h, w, y0 + p / hw - 1, x0 + p % hw - 1, tw, v);
+                load_octets(in, group * pl.nw * 16 + 8 * c8, img, h, w, y0 + p / hw - 1, x0 + p % hw - 1, tw, v);
                 stride = pl.in_stride;
                 dst = s_in + (size_t)(8 * c8) * stride + p;
             } else {
                 const int f = e - items_in, c8 = f % (cout / 8), p = f / (cout / 8);
-                load_octets(dpre, cout, 8 * c8, img, h, w, y0 + p / tw, x0 + p % tw, tw, v);
+                load_octets(dpre, 8 * c8, img, h, w, y0 + p / tw, x0 + p % tw, tw, v);
                 stride = pl.dp_stride;
                 dst = s_dp + (size_t)(8 * c8) * stride + p;
             }
@@ -352,86 +572,6 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(const float* __restrict__ par
     red[threadIdx.x] = acc;
     __syncthreads();
     if (q == 0 && e < row) grad[e] = ((red[threadIdx.x] + red[threadIdx.x + 64]) + red[threadIdx.x + 128]) + red[threadIdx.x + 192];
-}
-
-// ---------------------------------------------------------------------------
-// Elementwise and resampling kernels (NHWC bf16, fp32 arithmetic).
-// ---------------------------------------------------------------------------
-
-// d <- d * (y > 0): the ReLU's backward, in place.
-__global__ void k_relu_bwd(bf16* __restrict__ d, const bf16* __restrict__ y, size_t count) {
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += (size_t)gridDim.x * blockDim.x)
-        if (!(b2f(y[e]) > 0.0f)) d[e] = f2b(0.0f);
-}
-
-// 2x2 average pool: out[n][h/2][w/2][c].
-// 2x2 average pool and nearest-upsample + channel concat, eight channels
-// (16 bytes) per thread; channel counts are multiples of 16. The pool sums
-// the four taps in the same order for every channel.
-__global__ void k_pool(const bf16* __restrict__ in, int n, int h, int w, int c, bf16* __restrict__ out) {
-    const uint32_t c8 = (uint32_t)c / 8, w2 = (uint32_t)w / 2, h2 = (uint32_t)h / 2;
-    const uint32_t total = (uint32_t)n * h2 * w2 * c8;
-    for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += gridDim.x * blockDim.x) {
-        const uint32_t g = e % c8, p = e / c8;
-        const uint32_t x = p % w2, q = p / w2, y = q % h2, img = q / h2;
-        const bf16* b = in + (((size_t)img * h + 2 * y) * w + 2 * x) * c + 8 * g;
-        const bf16x8 v00 = *reinterpret_cast<const bf16x8*>(b);
-        const bf16x8 v01 = *reinterpret_cast<const bf16x8*>(b + c);
-        const bf16x8 v10 = *reinterpret_cast<const bf16x8*>(b + (size_t)w * c);
-        const bf16x8 v11 = *reinterpret_cast<const bf16x8*>(b + (size_t)w * c + c);
-        bf16x8 r;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) r[i] = f2b(0.25f * (b2f(v00[i]) + b2f(v01[i]) + b2f(v10[i]) + b2f(v11[i])));
-        *reinterpret_cast<bf16x8*>(out + (size_t)p * c + 8 * g) = r;
-    }
-}
-// Gradient through the pool plus the skip branch: out = up(dpool)/4 + dskip.
-__global__ void k_pool_bwd_add(const bf16* __restrict__ dpool, const bf16* __restrict__ dskip, int n, int h, int w,
-                               int c, bf16* __restrict__ out) {
-    const size_t total = (size_t)n * h * w * c;
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
-        const int ch = e % c;
-        size_t p = e / c;
-        const int x = p % w, y = (p / w) % h, img = p / ((size_t)w * h);
-        const float a = b2f(dpool[(((size_t)img * (h / 2) + y / 2) * (w / 2) + x / 2) * c + ch]);
-        out[e] = f2b(0.25f * a + (dskip ? b2f(dskip[e]) : 0.0f));
-    }
-}
-
-// Nearest 2x upsample of `low` (c1 channels) concatenated with `skip` (c2).
-__global__ void k_upcat(const bf16* __restrict__ low, int c1, const bf16* __restrict__ skip, int c2, int n, int h,
-                        int w, bf16* __restrict__ out) {
-    const uint32_t c8 = (uint32_t)(c1 + c2) / 8, l8 = (uint32_t)c1 / 8;
-    const uint32_t total = (uint32_t)n * h * w * c8;
-    for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += gridDim.x * blockDim.x) {
-        const uint32_t g = e % c8, p = e / c8;
-        const uint32_t x = p % (uint32_t)w, q = p / (uint32_t)w, y = q % (uint32_t)h, img = q / (uint32_t)h;
-        const bf16* src = g < l8 ? low + (((size_t)img * (h / 2) + y / 2) * (w / 2) + x / 2) * c1 + 8 * g
-                                 : skip + (size_t)p * c2 + 8 * (g - l8);
-        *reinterpret_cast<bf16x8*>(out + (size_t)e * 8) = *reinterpret_cast<const bf16x8*>(src);
-    }
-}
-// Backward of k_upcat: dlow sums its 2x2 block, dskip is a slice.
-__global__ void k_upcat_bwd(const bf16* __restrict__ dcat, int c1, int c2, int n, int h, int w, bf16* __restrict__ dlow,
-                            bf16* __restrict__ dskip) {
-    const int c = c1 + c2;
-    const size_t low_total = (size_t)n * (h / 2) * (w / 2) * c1;
-    const size_t skip_total = (size_t)n * h * w * c2;
-    const size_t total = low_total + skip_total;
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
-        if (e < low_total) {
-            const int ch = e % c1;
-            size_t p = e / c1;
-            const int x = p % (w / 2), y = (p / (w / 2)) % (h / 2), img = p / ((size_t)(w / 2) * (h / 2));
-            const bf16* b = dcat + (((size_t)img * h + 2 * y) * w + 2 * x) * c + ch;
-            dlow[e] = f2b(b2f(b[0]) + b2f(b[c]) + b2f(b[(size_t)w * c]) + b2f(b[(size_t)w * c + c]));
-        } else {
-            const size_t f = e - low_total;
-            const int ch = f % c2;
-            const size_t p = f / c2;
-            dskip[f] = dcat[p * c + c1 + ch];
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -595,43 +735,51 @@ size_t net_param_count() {
     return c;
 }
 
-template <int MT, int NT>
-static void launch_conv_t(hipStream_t s, const bf16* in, int cin, const bf16x8* f, const float* bias, int relu,
-                          bf16* out, int n, int h, int w) {
-    const int tiles = n * h * (w / (16 * NT));
-    hipLaunchKernelGGL((k_conv<MT, NT>), dim3((tiles + 3) / 4), dim3(256), 0, s, in, cin, f, bias, relu, out, n, h, w);
-}
+constexpr size_t CONV_LDS = 160 * 1024;  // LDS of a CU
 
-// Tiles per wave: 4 for 16 output channels, 2 above (more tiles cost
-// occupancy the weight reuse does not repay), fewer when the row width does
-// not divide.
-template <int MT>
-static void launch_conv_m(hipStream_t s, const bf16* in, int cin, const bf16x8* f, const float* bias, int relu,
-                          bf16* out, int n, int h, int w) {
-    constexpr int NT_MAX = MT == 1 ? 4 : 2;
-    if (NT_MAX == 4 && w % 64 == 0)
-        launch_conv_t<MT, NT_MAX>(s, in, cin, f, bias, relu, out, n, h, w);
-    else if (w % 32 == 0)
-        launch_conv_t<MT, 2>(s, in, cin, f, bias, relu, out, n, h, w);
-    else
-        launch_conv_t<MT, 1>(s, in, cin, f, bias, relu, out, n, h, w);
-}
-
-static lucida_status launch_conv(hipStream_t s, const bf16* in, int cin, int cout, const bf16* frag, const float* bias,
-                                 int relu, bf16* out, int n, int h, int w) {
-    const bf16x8* f = reinterpret_cast<const bf16x8*>(frag);
-    switch (cout / 16) {
-        case 1: launch_conv_m<1>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        case 2: launch_conv_m<2>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        case 3: launch_conv_m<3>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        case 4: launch_conv_m<4>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        case 5: launch_conv_m<5>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        case 6: launch_conv_m<6>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        case 7: launch_conv_m<7>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        case 10: launch_conv_m<10>(s, in, cin, f, bias, relu, out, n, h, w); break;
-        default: return set_error(LUCIDA_INVALID_ARG, "conv: unsupported output channel count");
+template <int MTW, int NT, int PF>
+static lucida_status launch_conv_t(hipStream_t s, int epi, ConvArgs a, int wm, int wn) {
+    a.wm = wm;
+    a.wn = wn;
+    a.rows = wn * (NT / 2);
+    a.tiles_x = (a.w + CONV_BW - 1) / CONV_BW;
+    a.tiles_y = (a.h + a.rows - 1) / a.rows;
+    const size_t lds = (size_t)(a.rows + 2) * CONV_LW * ((a.in.c_low + a.in.c) / 8 + 1) * 16;
+    if (lds > CONV_LDS || wm * wn > 8 || wm * MTW < a.mts)
+        return set_error(LUCIDA_INVALID_ARG, "conv: tile larger than a block");
+    const dim3 grid(a.n * a.tiles_x * a.tiles_y), block(64 * wm * wn);
+    switch (epi) {
+        case CONV_FWD: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_FWD>), grid, block, lds, s, a); break;
+        case CONV_FWD_POOL: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_FWD_POOL>), grid, block, lds, s, a); break;
+        case CONV_BWD: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_BWD>), grid, block, lds, s, a); break;
+        case CONV_BWD_SPLIT: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_BWD_SPLIT>), grid, block, lds, s, a); break;
+        default: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_BWD_UNPOOL>), grid, block, lds, s, a); break;
     }
     return LUCIDA_OK;
+}
+
+// The split by size. From 256 x 256 pixels a wave keeps all output tiles of 64 or
+// 128 pixels, as weights are then read least; 128 pixels only where two tiles and
+// few input channels leave LDS for it (80 channels: 217 us at 128 pixels, one
+// block a CU, 123 us at 64, both at 1024 x 1024). Below, and above five output
+// tiles, waves share the tiles in pairs, and below 128 x 128 one each, so that
+// the coarse levels still make enough waves (96 to 96 channels at 48 x 27: 16
+// us before with 81 waves, 13 us with 168).
+static lucida_status launch_conv(hipStream_t s, int epi, const ConvArgs& a) {
+    const int mt = a.mts;
+    const long px = (long)a.n * a.h * a.w;
+    if (mt > 10) return set_error(LUCIDA_INVALID_ARG, "conv: unsupported output channel count");
+    if (px < 256L * 256 || mt > 5) {
+        if (px < 128L * 128 && mt <= 8) return launch_conv_t<1, 4, 8>(s, epi, a, mt, 1);
+        return launch_conv_t<2, 4, 4>(s, epi, a, (mt + 1) / 2, mt <= 4 ? 2 : 1);
+    }
+    switch (mt) {
+        case 1: return launch_conv_t<1, 8, 4>(s, epi, a, 1, 4);
+        case 2: return a.in.c_low + a.in.c > 64 ? launch_conv_t<2, 4, 4>(s, epi, a, 1, 4) : launch_conv_t<2, 8, 2>(s, epi, a, 1, 4);
+        case 3: return launch_conv_t<3, 4, 4>(s, epi, a, 1, 4);
+        case 4: return launch_conv_t<4, 4, 2>(s, epi, a, 1, 4);
+        default: return launch_conv_t<5, 4, 2>(s, epi, a, 1, 4);
+    }
 }
 
 // How a layer's weight gradient is split. Tiles are 64 pixels wide where the
@@ -666,22 +814,22 @@ static WgradPlan plan_wgrad(int cin, int cout, int n, int h, int w) {
 }
 
 template <int MT>
-static lucida_status launch_wgrad_t(hipStream_t s, const bf16* in, int cin, const bf16* dpre, int n, int h, int w,
+static lucida_status launch_wgrad_t(hipStream_t s, const ConvSource& in, const bf16* dpre, int h, int w,
                                     const WgradPlan& p, float* part) {
     if (p.lds > WG_LDS) return set_error(LUCIDA_INVALID_ARG, "weight gradient: tile larger than LDS");
-    hipLaunchKernelGGL((k_wgrad<MT>), dim3(p.slices * p.groups), dim3(64 * p.nw * p.ksplit), p.lds, s, in, cin, dpre,
-                       n, h, w, p, part);
+    hipLaunchKernelGGL((k_wgrad<MT>), dim3(p.slices * p.groups), dim3(64 * p.nw * p.ksplit), p.lds, s, in,
+                       ConvSource{nullptr, dpre, 0, MT * 16}, h, w, p, part);
     return LUCIDA_OK;
 }
 
-static lucida_status launch_wgrad(hipStream_t s, const bf16* in, int cin, const bf16* dpre, int cout, int n, int h,
-                                  int w, const WgradPlan& p, float* part) {
+static lucida_status launch_wgrad(hipStream_t s, const ConvSource& in, const bf16* dpre, int cout, int h, int w,
+                                  const WgradPlan& p, float* part) {
     switch (cout / 16) {
-        case 1: return launch_wgrad_t<1>(s, in, cin, dpre, n, h, w, p, part);
-        case 2: return launch_wgrad_t<2>(s, in, cin, dpre, n, h, w, p, part);
-        case 3: return launch_wgrad_t<3>(s, in, cin, dpre, n, h, w, p, part);
-        case 4: return launch_wgrad_t<4>(s, in, cin, dpre, n, h, w, p, part);
-        case 6: return launch_wgrad_t<6>(s, in, cin, dpre, n, h, w, p, part);
+        case 1: return launch_wgrad_t<1>(s, in, dpre, h, w, p, part);
+        case 2: return launch_wgrad_t<2>(s, in, dpre, h, w, p, part);
+        case 3: return launch_wgrad_t<3>(s, in, dpre, h, w, p, part);
+        case 4: return launch_wgrad_t<4>(s, in, dpre, h, w, p, part);
+        case 6: return launch_wgrad_t<6>(s, in, dpre, h, w, p, part);
         default: return set_error(LUCIDA_INVALID_ARG, "weight gradient: unsupported output channel count");
     }
 }
@@ -719,7 +867,6 @@ struct ActPlan {
     size_t x;          // features [n][h][w][16]
     size_t l[15];      // outputs of layers 0..14
     size_t p0, p1, p2; // pooled skip0, skip1, skip2
-    size_t c2, c1, c0; // concatenations before layers 8, 10, 12
     size_t total;
 };
 
@@ -738,11 +885,24 @@ static ActPlan plan_acts(int n, int h, int w) {
     a.p0 = take(H[1], Wd[1], 32);
     a.p1 = take(H[2], Wd[2], 48);
     a.p2 = take(H[3], Wd[3], 64);
-    a.c2 = take(H[2], Wd[2], 160);
-    a.c1 = take(H[1], Wd[1], 112);
-    a.c0 = take(H[0], Wd[0], 80);
     a.total = off;
     return a;
+}
+
+// The input of layer li in the activations A: another layer's output, its
+// pooled output, or (layers 8, 10 and 12) the layer below upsampled and a skip.
+static ConvSource layer_source(const bf16* A, const ActPlan& a, int li) {
+    const int cin = kNetLayers[li].cin;
+    switch (li) {
+        case 0: return ConvSource{nullptr, A + a.x, 0, cin};
+        case 2: return ConvSource{nullptr, A + a.p0, 0, cin};
+        case 4: return ConvSource{nullptr, A + a.p1, 0, cin};
+        case 6: return ConvSource{nullptr, A + a.p2, 0, cin};
+        case 8: return ConvSource{A + a.l[7], A + a.l[5], kNetLayers[7].cout, kNetLayers[5].cout};
+        case 10: return ConvSource{A + a.l[9], A + a.l[3], kNetLayers[9].cout, kNetLayers[3].cout};
+        case 12: return ConvSource{A + a.l[11], A + a.l[1], kNetLayers[11].cout, kNetLayers[1].cout};
+        default: return ConvSource{nullptr, A + a.l[li - 1], 0, cin};
+    }
 }
 
 static lucida_status net_prep_frags(lucida_net* net) {
@@ -793,47 +953,27 @@ static lucida_status net_forward(lucida_net* net) {
     bf16* A = net->acts.as<bf16>();
     const float* P = net->params.as<float>();
     const bf16* F = net->frag_fwd.as<bf16>();
-    const int H[4] = {H0, H0 / 2, H0 / 4, H0 / 8}, Wd[4] = {W0, W0 / 2, W0 / 4, W0 / 8};
-    auto conv = [&](int li, size_t in_off, int lvl) {
+    for (int li = 0; li < kNetNumLayers; ++li) {
         const NetLayer& L = kNetLayers[li];
-        return launch_conv(s, A + in_off, L.cin, L.cout, F + net->frag_fwd_off[li],
-                           P + net->param_off[li] + (size_t)9 * L.cin * L.cout, L.relu, A + a.l[li], n, H[lvl],
-                           Wd[lvl]);
-    };
-    auto pool = [&](size_t in_off, int lvl, int c, size_t out_off) {
-        size_t total = (size_t)n * H[lvl + 1] * Wd[lvl + 1] * c / 8;
-        hipLaunchKernelGGL(k_pool, dim3(grid1(total)), dim3(256), 0, s, A + in_off, n, H[lvl], Wd[lvl], c,
-                           A + out_off);
-    };
-    auto upcat = [&](size_t low, int c1, size_t skip, int c2, int lvl, size_t out_off) {
-        size_t total = (size_t)n * H[lvl] * Wd[lvl] * (c1 + c2) / 8;
-        hipLaunchKernelGGL(k_upcat, dim3(grid1(total)), dim3(256), 0, s, A + low, c1, A + skip, c2, n, H[lvl],
-                           Wd[lvl], A + out_off);
-    };
-    lucida_status st;
-#define TRY(x)               \
-    if ((st = (x)) != LUCIDA_OK) return st;
-    TRY(conv(0, a.x, 0));
-    TRY(conv(1, a.l[0], 0));
-    pool(a.l[1], 0, 32, a.p0);
-    TRY(conv(2, a.p0, 1));
-    TRY(conv(3, a.l[2], 1));
-    pool(a.l[3], 1, 48, a.p1);
-    TRY(conv(4, a.p1, 2));
-    TRY(conv(5, a.l[4], 2));
-    pool(a.l[5], 2, 64, a.p2);
-    TRY(conv(6, a.p2, 3));
-    TRY(conv(7, a.l[6], 3));
-    upcat(a.l[7], 96, a.l[5], 64, 2, a.c2);
-    TRY(conv(8, a.c2, 2));
-    TRY(conv(9, a.l[8], 2));
-    upcat(a.l[9], 64, a.l[3], 48, 1, a.c1);
-    TRY(conv(10, a.c1, 1));
-    TRY(conv(11, a.l[10], 1));
-    upcat(a.l[11], 48, a.l[1], 32, 0, a.c0);
-    TRY(conv(12, a.c0, 0));
-    TRY(conv(13, a.l[12], 0));
-    TRY(conv(14, a.l[13], 0));
+        const int lvl = kNetLevel[li];
+        ConvArgs c{};
+        c.in = layer_source(A, a, li);
+        c.frag = reinterpret_cast<const bf16x8*>(F + net->frag_fwd_off[li]);
+        c.bias = P + net->param_off[li] + (size_t)9 * L.cin * L.cout;
+        c.relu = L.relu;
+        c.out = A + a.l[li];
+        c.n = n;
+        c.h = H0 >> lvl;
+        c.w = W0 >> lvl;
+        c.mts = L.cout / 16;
+        int epi = CONV_FWD;
+        if (li == 1 || li == 3 || li == 5) {  // pooled for the next level
+            epi = CONV_FWD_POOL;
+            c.out2 = A + (li == 1 ? a.p0 : li == 3 ? a.p1 : a.p2);
+        }
+        const lucida_status st = launch_conv(s, epi, c);
+        if (st != LUCIDA_OK) return st;
+    }
     LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
     return LUCIDA_OK;
 }
@@ -847,73 +987,53 @@ static lucida_status net_backward(lucida_net* net) {
     bf16* D = net->dacts.as<bf16>();
     float* G = net->grads.as<float>();
     const bf16* FB = net->frag_bwd.as<bf16>();
-    const int H[4] = {H0, H0 / 2, H0 / 4, H0 / 8}, Wd[4] = {W0, W0 / 2, W0 / 4, W0 / 8};
     // Every layer's W and b gradients are written whole by its k_wgrad_sum;
     // the partials buffer is sized for the layer with the most.
     WgradPlan wg[kNetNumLayers];
     size_t max_part = 0;
     for (int li = 0; li < kNetNumLayers; ++li) {
         const NetLayer& L = kNetLayers[li];
-        wg[li] = plan_wgrad(L.cin, L.cout, n, H[kNetLevel[li]], Wd[kNetLevel[li]]);
+        wg[li] = plan_wgrad(L.cin, L.cout, n, H0 >> kNetLevel[li], W0 >> kNetLevel[li]);
         max_part = std::max(max_part, (size_t)wg[li].slices * ((size_t)9 * L.cin * L.cout + L.cout));
     }
     if (max_part * 4 > net->wg_part.bytes) {
         LUCIDA_HIP(hipStreamSynchronize(s), LUCIDA_VALIDATION);
         LUCIDA_HIP(net->wg_part.ensure(max_part * 4), LUCIDA_OOM);
     }
-    lucida_status st;
-    // d(layer li's pre-activation) -> weight grads, and d(its input) into d_in.
-    auto layer_bwd = [&](int li, size_t in_off, int lvl, size_t d_in_off) -> lucida_status {
+    // Every gradient d(layer li) is stored after that layer's ReLU mask. A skip's
+    // gradient waits in the d slot of the layer before the skip (l[0], l[2] and
+    // l[4], written later) until the pooled branch's is added to it.
+    for (int li = kNetNumLayers - 1; li >= 0; --li) {
         const NetLayer& L = kNetLayers[li];
-        const size_t count = (size_t)n * H[lvl] * Wd[lvl] * L.cout;
-        if (L.relu)
-            hipLaunchKernelGGL(k_relu_bwd, dim3(grid1(count)), dim3(256), 0, s, D + a.l[li], A + a.l[li], count);
+        const int lvl = kNetLevel[li];
         const uint32_t row = (uint32_t)(9 * L.cin * L.cout + L.cout);  // the layer's W then b, as in `grads`
-        const lucida_status ws = launch_wgrad(s, A + in_off, L.cin, D + a.l[li], L.cout, n, H[lvl], Wd[lvl], wg[li],
-                                              net->wg_part.as<float>());
-        if (ws != LUCIDA_OK) return ws;
+        lucida_status st = launch_wgrad(s, layer_source(A, a, li), D + a.l[li], L.cout, H0 >> lvl, W0 >> lvl, wg[li],
+                                        net->wg_part.as<float>());
+        if (st != LUCIDA_OK) return st;
         hipLaunchKernelGGL(k_wgrad_sum, dim3((row + 63) / 64), dim3(256), 0, s, net->wg_part.as<float>(), row,
                            wg[li].slices, G + net->param_off[li]);
-        if (d_in_off == (size_t)-1) return LUCIDA_OK;
-        return launch_conv(s, D + a.l[li], L.cout, L.cin, FB + net->frag_bwd_off[li], nullptr, 0, D + d_in_off, n,
-                           H[lvl], Wd[lvl]);
-    };
-    auto upcat_bwd = [&](size_t dcat, int c1, int c2, int lvl, size_t dlow, size_t dskip) {
-        size_t total = (size_t)n * H[lvl] * Wd[lvl] * c2 + (size_t)n * H[lvl + 1] * Wd[lvl + 1] * c1;
-        hipLaunchKernelGGL(k_upcat_bwd, dim3(grid1(total)), dim3(256), 0, s, D + dcat, c1, c2, n, H[lvl], Wd[lvl],
-                           D + dlow, D + dskip);
-    };
-    auto pool_bwd_add = [&](size_t dpool, size_t dskip, int lvl, int c, size_t out) {
-        size_t total = (size_t)n * H[lvl] * Wd[lvl] * c;
-        hipLaunchKernelGGL(k_pool_bwd_add, dim3(grid1(total)), dim3(256), 0, s, D + dpool, D + dskip, n, H[lvl],
-                           Wd[lvl], c, D + out);
-    };
-    // Scratch gradient slots: the d of a concatenation input is computed into the
-    // cat buffers' d slots; d(skip) into the pooled buffers' d slots is not
-    // needed, the skip gradients go to a.l[*] d slots directly.
-    TRY(layer_bwd(14, a.l[13], 0, a.l[13]));
-    TRY(layer_bwd(13, a.l[12], 0, a.l[12]));
-    TRY(layer_bwd(12, a.c0, 0, a.c0));
-    // dcat0 -> d l[11] (low, 48 ch at level 1) and dskip0 (32 ch at level 0) parked in d l[0]'s slot
-    upcat_bwd(a.c0, 48, 32, 0, a.l[11], a.l[0]);
-    TRY(layer_bwd(11, a.l[10], 1, a.l[10]));
-    TRY(layer_bwd(10, a.c1, 1, a.c1));
-    upcat_bwd(a.c1, 64, 48, 1, a.l[9], a.l[2]);  // dskip1 parked in d l[2]'s slot
-    TRY(layer_bwd(9, a.l[8], 2, a.l[8]));
-    TRY(layer_bwd(8, a.c2, 2, a.c2));
-    upcat_bwd(a.c2, 96, 64, 2, a.l[7], a.l[4]);  // dskip2 parked in d l[4]'s slot
-    TRY(layer_bwd(7, a.l[6], 3, a.l[6]));
-    TRY(layer_bwd(6, a.p2, 3, a.p2));
-    pool_bwd_add(a.p2, a.l[4], 2, 64, a.l[5]);   // d l[5] = pool_bwd(d p2) + dskip2
-    TRY(layer_bwd(5, a.l[4], 2, a.l[4]));
-    TRY(layer_bwd(4, a.p1, 2, a.p1));
-    pool_bwd_add(a.p1, a.l[2], 1, 48, a.l[3]);   // d l[3] = pool_bwd(d p1) + dskip1
-    TRY(layer_bwd(3, a.l[2], 1, a.l[2]));
-    TRY(layer_bwd(2, a.p0, 1, a.p0));
-    pool_bwd_add(a.p0, a.l[0], 0, 32, a.l[1]);   // d l[1] = pool_bwd(d p0) + dskip0
-    TRY(layer_bwd(1, a.l[0], 0, a.l[0]));
-    TRY(layer_bwd(0, a.x, 0, (size_t)-1));
-#undef TRY
+        if (li == 0) break;
+        ConvArgs c{};
+        c.in = ConvSource{nullptr, D + a.l[li], 0, L.cout};
+        c.frag = reinterpret_cast<const bf16x8*>(FB + net->frag_bwd_off[li]);
+        c.n = n;
+        c.h = H0 >> lvl;
+        c.w = W0 >> lvl;
+        c.mts = L.cin / 16;
+        c.out = D + a.l[li - 1];
+        c.mask = A + a.l[li - 1];
+        int epi = CONV_BWD;
+        if (li == 8 || li == 10 || li == 12) {  // the upsampled layer below, and a skip
+            epi = CONV_BWD_SPLIT;
+            c.c_split = kNetLayers[li - 1].cout;
+            c.out2 = D + a.l[12 - li];
+        } else if (li == 2 || li == 4 || li == 6) {
+            epi = CONV_BWD_UNPOOL;
+            c.add = D + a.l[li - 2];
+        }
+        st = launch_conv(s, epi, c);
+        if (st != LUCIDA_OK) return st;
+    }
     LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
     return LUCIDA_OK;
 }

@@ -55,3 +55,46 @@ def test_weight_gradients_of_stored_tensors(gpu, w, h, n):
         off += 9 * ci * co
         assert np.all(np.abs(grads[off:off + co] - dm.sum(0)) <= 2.0 ** -16 * np.abs(dm).sum(0) + 1e-30), i
         off += co
+
+
+@pytest.mark.parametrize("w,h,n", SHAPES)
+def test_convolutions_of_stored_tensors(gpu, w, h, n):
+    """Every layer's output, and every gradient that the next layer's input
+    gradient, pools and concatenations make of it, recomputed in float64 from
+    the tensors the device stored. BF16 rounds to 2^-9 of the value; a flip of
+    that rounding, or one more rounding of a summand, adds as much again, and
+    the FP32 sums of at most 1440 products 2^-13 of the terms' magnitude."""
+    net, acts = run_backward(gpu, w, h, n, 71)
+    params = N.unpack(net.params().astype(np.float64))
+    for i, (ci, co, relu) in enumerate(N.LAYERS):
+        wt, b = N.to_bf16(params[i][0]), params[i][1]
+        want = N.conv3x3(acts[LAYER_INPUT[i]], wt, b)
+        size = N.conv3x3(np.abs(acts[LAYER_INPUT[i]]), np.abs(wt), np.abs(b))
+        if relu:
+            want = np.maximum(want, 0)
+        got = acts[f"l{i}"]
+        assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -13 * size + 1e-30), i
+
+    def input_grad(i):
+        d = net.tensor(i + 1, gradient=True).astype(np.float64)
+        back = N.to_bf16(params[i][0])[::-1].transpose(0, 2, 1)
+        return N.conv3x3(d, back), N.conv3x3(np.abs(d), np.abs(back))
+
+    skips = {}
+    for i in range(14, 0, -1):
+        g, size = input_grad(i)
+        slack = 2.0 ** -8 * np.abs(g) + 2.0 ** -13 * size
+        below = i - 1
+        if i in (8, 10, 12):
+            c = N.LAYERS[below][1]
+            skips[i] = (g[..., c:], slack[..., c:])
+            quads = lambda t: sum(t[:, y::2, x::2, :c] for y in (0, 1) for x in (0, 1))
+            g, slack = quads(g), quads(slack)
+        elif i in (2, 4, 6):
+            up = lambda t: t.repeat(2, 1).repeat(2, 2)
+            sg, ss = skips[{2: 12, 4: 10, 6: 8}[i]]
+            g, slack = 0.25 * up(g) + sg, 0.25 * up(slack) + ss
+        mask = acts[f"l{below}"] > 0
+        got = net.tensor(below + 1, gradient=True).astype(np.float64)
+        assert np.all(got[~mask] == 0), i
+        assert np.all(np.abs(got - g * mask) <= (slack + 2.0 ** -8 * np.abs(g)) * mask + 1e-30), i
