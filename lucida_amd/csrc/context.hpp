@@ -179,8 +179,9 @@ lucida_status build_prim_planes(lucida_ctx* ctx, lucida_scene* scene);
 // Fills scene->tri_edges from its (final, leaf-ordered) triangles.
 lucida_status build_tri_edges(lucida_ctx* ctx, lucida_scene* scene);
 // A-trous filter (atrous.hip) without the final wait: reserve the planes for
-// the largest film first, then queue filters on the context's stream.
+// the films' pixels together first, then queue their filters on the context's
+// stream, film k into out[k].
 lucida_status atrous_reserve(lucida_ctx* ctx, size_t pixels);
-void atrous_enqueue(lucida_ctx* ctx, const GpuAccum* in, uint32_t w, uint32_t h, const lucida_denoise_params& params,
-                    GpuAccum* out);
+void atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuAccum* const* out, size_t count,
+                    const lucida_denoise_params& params);
 }  // namespace lucida

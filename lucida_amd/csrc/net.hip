@@ -586,11 +586,25 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(const float* __restrict__ par
 // `target` non-null also writes the target log1p(ref radiance / albedo) (3
 // floats per pixel) from the reference film, demodulated by the INPUT film's
 // albedo so inference can remodulate with the same guide.
-__global__ void k_features(const GpuAccum* __restrict__ film, const GpuAccum* __restrict__ base,
-                           const GpuAccum* __restrict__ ref, int fw, int x0, int y0, int cw, int ch, int img,
-                           bf16* __restrict__ feat, float* __restrict__ base_log, float* __restrict__ target) {
+//
+// One launch serves up to FEATURE_FILMS films (blockIdx.z): each one's filtered
+// and reference films, row width and crop origin, and its place in the batch.
+constexpr int FEATURE_FILMS = 16;
+struct FeatureFilm {
+    const GpuAccum *film, *base, *ref;
+    int fw, x0, y0, img;
+};
+struct FeatureFilms {
+    FeatureFilm film[FEATURE_FILMS];
+};
+
+__global__ void k_features(FeatureFilms films, int cw, int ch, bf16* __restrict__ feat, float* __restrict__ base_log,
+                           float* __restrict__ target) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
     if (x >= cw || y >= ch) return;
+    const FeatureFilm& F = films.film[blockIdx.z];
+    const GpuAccum *film = F.film, *base = F.base, *ref = F.ref;
+    const int fw = F.fw, x0 = F.x0, y0 = F.y0, img = F.img;
     const size_t src = (size_t)(y0 + y) * fw + (x0 + x);
     const float4* a = reinterpret_cast<const float4*>(film + src);
     const float4 a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
@@ -711,6 +725,10 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ grad, fl
 // The a-trous filter the network corrects: DenoiseParams' defaults
 // (crates/core/src/denoise.rs:62-94).
 const lucida_denoise_params kAtrousDefaults = {4u, 64.0f, 0.08f, 4.0f, 0.1f};
+
+// Films filtered together for a batch's features, by their pixels: enough to
+// fill the device, while the filter's planes and results stay near 500 MB.
+constexpr size_t NET_FILTER_PIXELS = (size_t)1 << 22;
 
 inline unsigned grid1(size_t n, int block = 256) {
     size_t g = (n + block - 1) / block;
@@ -852,7 +870,7 @@ struct lucida_net {
     DevBuf frag_fwd, frag_bwd;             // bf16 fragments
     size_t frag_fwd_off[kNetNumLayers], frag_bwd_off[kNetNumLayers], param_off[kNetNumLayers];
     DevBuf acts, dacts, target, loss_partial;
-    DevBuf base;  // a-trous estimate of the film being loaded (Accum-shaped)
+    DevBuf base;  // a-trous estimates of the films being loaded (Accum-shaped)
     DevBuf base_log;  // its log1p(estimate / albedo) per pixel of the batch, FP32 (3 floats)
     size_t act_capacity = 0;
     uint32_t step = 0;
@@ -1148,9 +1166,20 @@ static lucida_status load_batch(lucida_net* net, const lucida_film* const* input
     }
     lucida_status st = net_ensure_acts(net, (int)count, (int)h, (int)w);
     if (st != LUCIDA_OK) return st;
-    size_t max_pixels = 0;
-    for (uint32_t k = 0; k < count; ++k)
-        max_pixels = std::max<size_t>(max_pixels, (size_t)inputs[k]->width * inputs[k]->height);
+    // Whole films are filtered (crops then see the filter's real neighbourhood),
+    // as many together as make NET_FILTER_PIXELS, each into its part of `base`.
+    auto pixels_of = [&](uint32_t k) { return (size_t)inputs[k]->width * inputs[k]->height; };
+    auto group_end = [&](uint32_t first, size_t* pixels) {
+        uint32_t k = first;
+        *pixels = 0;
+        while (k < count && (k == first || *pixels + pixels_of(k) <= NET_FILTER_PIXELS)) *pixels += pixels_of(k++);
+        return k;
+    };
+    size_t max_pixels = 0, group = 0;
+    for (uint32_t k = 0; k < count;) {
+        k = group_end(k, &group);
+        max_pixels = std::max(max_pixels, group);
+    }
     if (max_pixels * sizeof(GpuAccum) > net->base.bytes) {
         LUCIDA_HIP(hipStreamSynchronize(net->ctx->stream), LUCIDA_VALIDATION);
         LUCIDA_HIP(net->base.ensure(max_pixels * sizeof(GpuAccum)), LUCIDA_OOM);
@@ -1159,16 +1188,27 @@ static lucida_status load_batch(lucida_net* net, const lucida_film* const* input
     if (st != LUCIDA_OK) return st;
     const ActPlan a = plan_acts(net->n, net->h, net->w);
     bf16* X = net->acts.as<bf16>() + a.x;
-    for (uint32_t k = 0; k < count; ++k) {
-        const lucida_film* f = inputs[k];
-        const uint32_t cx = x0 ? x0[k] : 0, cy = y0 ? y0[k] : 0;
-        // The whole film is filtered (crops then see the filter's real
-        // neighbourhood); stream order keeps one scratch film enough.
-        atrous_enqueue(net->ctx, f->accum, f->width, f->height, kAtrousDefaults, net->base.as<GpuAccum>());
-        hipLaunchKernelGGL(k_features, dim3((w + 127) / 128, h), dim3(128), 0, net->ctx->stream, f->accum,
-                           net->base.as<GpuAccum>(), refs ? refs[k]->accum : nullptr, (int)f->width, (int)cx, (int)cy,
-                           (int)w, (int)h, (int)k, X, net->base_log.as<float>(),
-                           refs ? net->target.as<float>() : nullptr);
+    std::vector<GpuAccum*> filtered;
+    for (uint32_t first = 0; first < count;) {
+        const uint32_t end = group_end(first, &group);
+        filtered.clear();
+        GpuAccum* at = net->base.as<GpuAccum>();
+        for (uint32_t k = first; k < end; ++k) {
+            filtered.push_back(at);
+            at += pixels_of(k);
+        }
+        atrous_enqueue(net->ctx, inputs + first, filtered.data(), end - first, kAtrousDefaults);
+        for (uint32_t f0 = first; f0 < end; f0 += FEATURE_FILMS) {
+            FeatureFilms ff{};
+            const uint32_t n = std::min<uint32_t>(FEATURE_FILMS, end - f0);
+            for (uint32_t k = 0; k < n; ++k)
+                ff.film[k] = FeatureFilm{inputs[f0 + k]->accum, filtered[f0 + k - first],
+                                         refs ? refs[f0 + k]->accum : nullptr, (int)inputs[f0 + k]->width,
+                                         x0 ? (int)x0[f0 + k] : 0, y0 ? (int)y0[f0 + k] : 0, (int)(f0 + k)};
+            hipLaunchKernelGGL(k_features, dim3((w + 127) / 128, h, n), dim3(128), 0, net->ctx->stream, ff, (int)w,
+                               (int)h, X, net->base_log.as<float>(), refs ? net->target.as<float>() : nullptr);
+        }
+        first = end;
     }
     LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
     return LUCIDA_OK;
