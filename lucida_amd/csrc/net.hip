@@ -102,16 +102,20 @@ __global__ void k_wprep(const float* __restrict__ W, int cin, int cout, int tran
 //                   pixels, masked
 // Each rounds to BF16 where a separate pass would have read BF16, so results are
 // the same bit for bit.
-// What bounds it: staging and products share a block's time without overlapping
-// inside it, so it lives from the two or three blocks that a CU's LDS holds.
-// Inference of 1024 x 1024: the fifteen layers with their pools and
-// concatenations took 858 us with every wave reading its operands from L2 for
-// 32 pixels and the passes apart, 535 us so; the four passes of a training
-// step's backward (masks, pools, concatenations) took 400 us and are gone.
+// What bounds it: staging, products and stores share a block's time without
+// overlapping inside it, so it lives from the two or three blocks that a CU's
+// LDS holds (80 -> 32 channels at 1024 x 1024: 103 us, 57 without staging, 74
+// without products). Inference of 1024 x 1024: the fifteen layers with their
+// pools and concatenations took 858 us with every wave reading its operands
+// from L2 for 32 pixels and the passes apart, and take 470 us so; the passes of
+// a training step's backward (masks, pools, concatenations) took 400 us and are
+// gone. K loops with a branch per chunk cost 65 us more: every chunk then
+// waited for the newest weights.
 // ---------------------------------------------------------------------------
 enum { CONV_FWD, CONV_FWD_POOL, CONV_BWD, CONV_BWD_SPLIT, CONV_BWD_UNPOOL };
 constexpr int CONV_BW = 32;           // a block's pixels per row
 constexpr int CONV_LW = CONV_BW + 2;  // with the halo
+constexpr int CONV_MAX_KBS = 90;      // K-blocks of 160 input channels
 constexpr int CONV_STAGE = 10;        // loads in flight a thread while staging
 
 // An NHWC tensor of c_low + c channels: the first c_low from `low` at half the
@@ -240,10 +244,57 @@ __device__ inline void conv_emit(const ConvArgs& a, int img, int y0, int x0, int
         }
 }
 
+// Stages rows by - 1 .. by + rows and columns x0 - 1 .. x0 + CONV_BW of image img
+// in `lds`: consecutive threads take consecutive octets of the tile's pixels,
+// CONV_STAGE loads in flight a thread.
+template <bool CAT>
+__device__ inline void conv_stage(const ConvArgs& a, int img, int by, int x0, uint4* lds) {
+    const int c = a.in.c, c_low = CAT ? a.in.c_low : 0;
+    const int octs = (c_low + c) / 8, S = octs + 1, lrows = a.rows + 2;
+    const bf16* lowi = CAT ? a.in.low + (size_t)img * (a.h / 2) * (a.w / 2) * c_low : nullptr;
+    const bf16* srci = a.in.src + (size_t)img * a.h * a.w * c;
+    const int step_o = blockDim.x % octs, step_p = blockDim.x / octs;
+    int o = threadIdx.x % octs, p = threadIdx.x / octs;
+    int ry = p / CONV_LW, px = p - ry * CONV_LW;
+    while (ry < lrows) {
+        uint4 v[CONV_STAGE];
+        int at[CONV_STAGE];
+#pragma unroll
+        for (int k = 0; k < CONV_STAGE; ++k) {
+            const int x = x0 - 1 + px, y = by - 1 + ry;
+            at[k] = ry < lrows ? (ry * CONV_LW + px) * S + o : -1;
+            v[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (ry < lrows && x >= 0 && x < a.w && y >= 0 && y < a.h) {
+                const bf16* q;
+                if (CAT && 8 * o < c_low)
+                    q = lowi + (((uint32_t)(y >> 1) * (a.w / 2) + (x >> 1)) * c_low + 8 * o);
+                else
+                    q = srci + (((uint32_t)y * a.w + x) * c + 8 * o - c_low);
+                v[k] = *reinterpret_cast<const uint4*>(q);
+            }
+            o += step_o;
+            px += step_p;
+            if (o >= octs) {
+                o -= octs;
+                ++px;
+            }
+            while (px >= CONV_LW) {
+                px -= CONV_LW;
+                ++ry;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < CONV_STAGE; ++k)
+            if (at[k] >= 0) lds[at[k]] = v[k];
+    }
+}
+
 template <int MTW, int NT, int PF, int EPI>
 __global__ __launch_bounds__(512) void k_conv(ConvArgs a) {
+    static_assert(PF % 2 == 0, "the input fragments alternate between two buffers");
     extern __shared__ uint4 cv_lds[];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    __shared__ int s_off[CONV_MAX_KBS + 1];  // K-block -> octet offset in the tile
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wmi = wv % a.wm, wni = wv / a.wm;
     const int g = lane >> 4, r = lane & 15;
     const int tile = xcd_order(blockIdx.x, gridDim.x);
@@ -251,106 +302,85 @@ __global__ __launch_bounds__(512) void k_conv(ConvArgs a) {
     const int by = (rest % a.tiles_y) * a.rows, img = rest / a.tiles_y;
     const int x0 = tx * CONV_BW;
     const int cin = a.in.c_low + a.in.c;
-    const int octs = cin / 8, S = octs + 1;
-    // Stage: consecutive threads take consecutive octets of the tile's pixels,
-    // CONV_STAGE loads in flight a thread.
-    {
-        const bf16* lowi = a.in.low + (size_t)img * (a.h / 2) * (a.w / 2) * a.in.c_low;
-        const bf16* srci = a.in.src + (size_t)img * a.h * a.w * a.in.c;
-        const int step_o = blockDim.x % octs, step_p = blockDim.x / octs;
-        int o = threadIdx.x % octs, p = threadIdx.x / octs;
-        int ry = p / CONV_LW, px = p - ry * CONV_LW;
-        while (ry < a.rows + 2) {
-            uint4 v[CONV_STAGE];
-            int at[CONV_STAGE];
-#pragma unroll
-            for (int k = 0; k < CONV_STAGE; ++k) {
-                const int x = x0 - 1 + px, y = by - 1 + ry;
-                at[k] = ry < a.rows + 2 ? (ry * CONV_LW + px) * S + o : -1;
-                v[k] = make_uint4(0u, 0u, 0u, 0u);
-                if (at[k] >= 0 && x >= 0 && x < a.w && y >= 0 && y < a.h) {
-                    const bool low = 8 * o < a.in.c_low;
-                    const uint32_t i = low ? ((uint32_t)(y >> 1) * (a.w / 2) + (x >> 1)) * a.in.c_low + 8 * o
-                                           : ((uint32_t)y * a.w + x) * a.in.c + 8 * o - a.in.c_low;
-                    v[k] = *reinterpret_cast<const uint4*>((low ? lowi : srci) + i);
-                }
-                o += step_o;
-                px += step_p;
-                if (o >= octs) {
-                    o -= octs;
-                    ++px;
-                }
-                while (px >= CONV_LW) {
-                    px -= CONV_LW;
-                    ++ry;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < CONV_STAGE; ++k)
-                if (at[k] >= 0) cv_lds[at[k]] = v[k];
-        }
-    }
+    const int S = cin / 8 + 1;
     const int cbs = cin / 16, kbs = 9 * cbs, chunks = (kbs + 1) / 2;
     const int mt0 = wmi * MTW;
-    const bf16x8* fp[MTW];  // the wave's fragments of a chunk (a tile past the last repeats it)
+    // the wave's weight fragments of a chunk (a tile past the last repeats it)
+    auto weights = [&](int c, bf16x8(&to)[MTW]) {
 #pragma unroll
-    for (int m = 0; m < MTW; ++m) fp[m] = a.frag + (size_t)min(mt0 + m, a.mts - 1) * 64 + lane;
-    const size_t fstep = (size_t)a.mts * 64;
+        for (int m = 0; m < MTW; ++m) to[m] = a.frag[((size_t)c * a.mts + min(mt0 + m, a.mts - 1)) * 64 + lane];
+    };
     bf16x8 av[PF][MTW];
 #pragma unroll
-    for (int i = 0; i < PF; ++i)
-#pragma unroll
-        for (int m = 0; m < MTW; ++m) av[i][m] = fp[m][fstep * min(i, chunks - 1)];
+    for (int i = 0; i < PF; ++i) weights(min(i, chunks - 1), av[i]);
+    for (int kb = threadIdx.x; kb <= kbs; kb += blockDim.x) {
+        const int tap = kb == kbs ? 8 : kb / cbs, cb = kb == kbs ? 0 : kb % cbs;
+        s_off[kb] = (tap / 3 * CONV_LW + tap % 3) * S + 2 * cb;
+    }
+    if (a.in.c_low)
+        conv_stage<true>(a, img, by, x0, cv_lds);
+    else
+        conv_stage<false>(a, img, by, x0, cv_lds);
     f32x4 acc[NT][MTW];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int m = 0; m < MTW; ++m) acc[t][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const int wrow = wni * (NT / 2);  // the wave's first row in the tile
-    const uint4* bp = cv_lds + (size_t)(wrow * CONV_LW + r) * S + (g & 1);
-    int tap0 = 0, cb0 = 0;  // of the chunk's first K-block
+    const uint4* bp[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) bp[t] = cv_lds + ((wrow + t / 2) * CONV_LW + 16 * (t % 2) + r) * S + (g & 1);
     __syncthreads();
-    for (int c0 = 0; c0 < chunks; c0 += PF) {
+    // The offsets of the lane's K-blocks are read a group of chunks ahead, the
+    // input fragments one chunk ahead.
+    int off[PF], off_next[PF];
+    auto offsets = [&](int c0, int(&to)[PF]) {
+#pragma unroll
+        for (int i = 0; i < PF; ++i) to[i] = s_off[min(2 * (c0 + i) + (g >> 1), kbs)];
+    };
+    uint4 bv[2][NT];
+    offsets(0, off);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) bv[0][t] = bp[t][off[0]];
+    auto products = [&](const bf16x8(&w)[MTW], const uint4(&x)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int m = 0; m < MTW; ++m)
+                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[m], __builtin_bit_cast(bf16x8, x[t]), acc[t][m],
+                                                                    0, 0, 0);
+    };
+    // Whole groups without a branch: after one the compiler would wait for
+    // every load in flight, the next group's weights among them.
+    int c0 = 0;
+    for (; c0 + PF < chunks; c0 += PF) {
+        offsets(c0 + PF, off_next);
 #pragma unroll
         for (int i = 0; i < PF; ++i) {
-            const int c = c0 + i;
-            if (c < chunks) {
-                // the chunk's two K-blocks; an odd count's missing last one has
-                // zero weights and reads zeros
-                int tap1 = tap0, cb1 = cb0 + 1;
-                if (cb1 == cbs) {
-                    cb1 = 0;
-                    ++tap1;
-                }
-                const bool pad = tap1 == 9;
-                const int off0 = (tap0 / 3 * CONV_LW + tap0 % 3) * S + 2 * cb0;
-                const int off1 = pad ? off0 : (tap1 / 3 * CONV_LW + tap1 % 3) * S + 2 * cb1;
-                const uint4* q = bp + (g < 2 ? off0 : off1);
-                uint4 bv[NT];
+            const int on = i + 1 < PF ? off[i + 1 < PF ? i + 1 : 0] : off_next[0];
 #pragma unroll
-                for (int t = 0; t < NT; ++t) bv[t] = q[((t / 2) * CONV_LW + 16 * (t % 2)) * S];
-                if (pad && g >= 2) {
+            for (int t = 0; t < NT; ++t) bv[(i + 1) & 1][t] = bp[t][on];
+            products(av[i], bv[i & 1]);
+            weights(min(c0 + i + PF, chunks - 1), av[i]);
+        }
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) bv[t] = make_uint4(0u, 0u, 0u, 0u);
-                }
+        for (int i = 0; i < PF; ++i) off[i] = off_next[i];
+    }
+    // The last group, whose weights are loaded. An odd count's missing last
+    // K-block has zero weights and takes zeros.
 #pragma unroll
-                for (int t = 0; t < NT; ++t)
+    for (int i = 0; i < PF; ++i) {
+        const int c = c0 + i;
+        if (c < chunks) {
+            if (i + 1 < PF && c + 1 < chunks) {
 #pragma unroll
-                    for (int m = 0; m < MTW; ++m)
-                        acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i][m], __builtin_bit_cast(bf16x8, bv[t]),
-                                                                            acc[t][m], 0, 0, 0);
-                cb0 = cb1 + 1;
-                tap0 = tap1;
-                if (cb0 == cbs) {
-                    cb0 = 0;
-                    ++tap0;
-                }
-                const int cn = c + PF;
-                if (cn < chunks) {
-#pragma unroll
-                    for (int m = 0; m < MTW; ++m) av[i][m] = fp[m][fstep * cn];
-                }
+                for (int t = 0; t < NT; ++t) bv[(i + 1) & 1][t] = bp[t][off[i + 1 < PF ? i + 1 : 0]];
             }
+            if (2 * c + 1 == kbs && g >= 2) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) bv[i & 1][t] = make_uint4(0u, 0u, 0u, 0u);
+            }
+            products(av[i], bv[i & 1]);
         }
     }
     // D: lane holds rows 4g + j of each output tile, pixel column r.
@@ -753,7 +783,7 @@ size_t net_param_count() {
     return c;
 }
 
-constexpr size_t CONV_LDS = 160 * 1024;  // LDS of a CU
+constexpr size_t CONV_LDS = 160 * 1024 - 512;  // LDS of a CU, less the offset table
 
 template <int MTW, int NT, int PF>
 static lucida_status launch_conv_t(hipStream_t s, int epi, ConvArgs a, int wm, int wn) {
@@ -763,7 +793,7 @@ static lucida_status launch_conv_t(hipStream_t s, int epi, ConvArgs a, int wm, i
     a.tiles_x = (a.w + CONV_BW - 1) / CONV_BW;
     a.tiles_y = (a.h + a.rows - 1) / a.rows;
     const size_t lds = (size_t)(a.rows + 2) * CONV_LW * ((a.in.c_low + a.in.c) / 8 + 1) * 16;
-    if (lds > CONV_LDS || wm * wn > 8 || wm * MTW < a.mts)
+    if (lds > CONV_LDS || wm * wn > 8 || wm * MTW < a.mts || a.in.c_low + a.in.c > CONV_MAX_KBS / 9 * 16)
         return set_error(LUCIDA_INVALID_ARG, "conv: tile larger than a block");
     const dim3 grid(a.n * a.tiles_x * a.tiles_y), block(64 * wm * wn);
     switch (epi) {
@@ -779,10 +809,12 @@ static lucida_status launch_conv_t(hipStream_t s, int epi, ConvArgs a, int wm, i
 // The split by size. From 256 x 256 pixels a wave keeps all output tiles of 64 or
 // 128 pixels, as weights are then read least; 128 pixels only where two tiles and
 // few input channels leave LDS for it (80 channels: 217 us at 128 pixels, one
-// block a CU, 123 us at 64, both at 1024 x 1024). Below, and above five output
-// tiles, waves share the tiles in pairs, and below 128 x 128 one each, so that
-// the coarse levels still make enough waves (96 to 96 channels at 48 x 27: 16
-// us before with 81 waves, 13 us with 168).
+// block a CU, 123 us at 64, both at 1024 x 1024); blocks of two waves instead
+// of four lose more to the halo than they gain (513 us for all layers against
+// 469). Below, and above five output tiles, waves share the tiles in pairs,
+// and below 128 x 128 one each, so that the coarse levels still make enough
+// waves (96 to 96 channels at 48 x 27: 16 us with 81 waves that keep all
+// tiles, 8 us with 168).
 static lucida_status launch_conv(hipStream_t s, int epi, const ConvArgs& a) {
     const int mt = a.mts;
     const long px = (long)a.n * a.h * a.w;
