@@ -1428,6 +1428,108 @@ __global__ __launch_bounds__(TRACE_WG) void k_megakernel(SceneView sc, const Gpu
 }
 
 // ---------------------------------------------------------------------------
+// PATHS: a whole path per thread in one launch, from its camera ray to its end:
+// the closest-hit walk, shade_bounce, the shadow ray's walk, the next ray, with
+// the wavefront stages' own code and in their order, so a path's radiance and
+// guides are theirs bit for bit. Unlike the megakernel, samples are threads of
+// their own and RESOLVE sums them.
+//
+// Too few paths to fill the device make every stage last as long as its
+// slowest ray, and those add up over the bounces, with a launch and an event
+// between streams for each; one launch lasts as long as its slowest path. With
+// more paths the stages win: they regroup the live paths, and keep up to eight
+// waves on a SIMD where the whole path's registers allow two. The line is what
+// the device holds at once, two waves on each SIMD of its CUs (131,072 paths):
+// up to it a render got faster on every scene, above it slower on most. ms in
+// stages / as paths, at 57,600, 131,044 and 163,840 paths:
+//   box-c1 (10 triangles)      0.40 / 0.21   0.44 / 0.22   0.43 / 0.34
+//   cornell-mesh (10,252)      1.02 / 0.91   1.14 / 1.04   1.12 / 1.25
+//   sphere-c2 (82,944)         1.62 / 1.30   1.76 / 1.31   1.84 / 2.11
+//   sphere-c2 (1,049,844)      2.68 / 1.71   3.00 / 1.79   3.05 / 2.73
+//   instances-c3 (4,096)       5.52 / 4.32   6.04 / 5.01   6.01 / 5.29
+//   bvh-stress (368,640)       1.47 / 1.41   1.73 / 1.52   1.64 / 2.01
+// ---------------------------------------------------------------------------
+constexpr size_t PATHS_WAVES_PER_CU = 8;
+
+template <int MODE>
+__global__ __launch_bounds__(TRACE_WG) void k_paths(SceneView sc, const GpuUniforms* __restrict__ U, Planes p,
+                                                    Band band) {
+    __shared__ uint32_t stack_mem[LDS_STACK * TRACE_WG];
+    const uint32_t i = blockIdx.x * TRACE_WG + threadIdx.x;
+    const GpuUniforms& u = *U;
+    uint32_t visits = 0, tests = 0, overflow = 0, rays = 0, shadow_rays = 0;
+    if (i < band.count * u.samples_per_launch) {
+        RayStack st = make_stack(stack_mem, p.spill, MODE == TRAV_BINARY ? STACK : INST_STACK);
+        PathRegs P;
+        camera_ray(u, band.first + i % band.count, u.sample_offset + i / band.count, &P.s, &P.origin, &P.dir);
+        P.throughput = v3(1.0f, 1.0f, 1.0f);
+        P.radiance = v3(0.0f, 0.0f, 0.0f);
+        P.prev_position = P.origin;
+        P.prev_bsdf_pdf = 0.0f;
+        P.depth = 0;
+        float4 gal = make_float4(0.0f, 0.0f, 0.0f, 0.0f), gnr = gal;
+        for (;;) {
+            // EXTEND
+            ++rays;
+            const V3 o = P.origin, d = P.dir;
+            float best_t = T_MAX;
+            uint32_t best = MISS;
+            analytic_closest(sc, o, d, &best_t, &best);
+            float t = 0.0f, hu = 0.0f, hv = 0.0f;
+            uint32_t tri = 0, inst = 0;
+            const bool two_level = MODE == TRAV_INSTANCED && sc.num_instances;
+            bool th;
+            if (two_level)
+                th = traverse_instances<false>(sc, st, o, d, T_MIN, best_t, &t, &hu, &hv, &tri, &inst, &visits, &tests,
+                                               &overflow);
+            else
+                th = traverse<false>(sc, st, 0, o, d, T_MIN, best_t, &t, &hu, &hv, &tri, &visits, &tests, &overflow);
+            float4 hit;
+            if (th) hit = make_float4(t, hu, hv, __uint_as_float(tri));
+            else if (best != MISS) hit = make_float4(best_t, 0.0f, 0.0f, __uint_as_float(ANALYTIC | best));
+            else hit = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(MISS));
+            // SHADE
+            bool shadow, guide;
+            ShadowRay sr;
+            float4 g0, g1;
+            const bool alive = shade_bounce(sc, u, hit, two_level ? inst : 0u, P, shadow, sr, guide, g0, g1);
+            if (guide) {
+                gal = g0;
+                gnr = g1;
+            }
+            // CONNECT
+            if (shadow) {
+                ++shadow_rays;
+                bool blocked = analytic_any(sc, sr.o, sr.d, sr.t_max);
+                if (!blocked) {
+                    float tt, uu, vv;
+                    uint32_t tri2, inst2;
+                    if (two_level)
+                        blocked = traverse_instances<true>(sc, st, sr.o, sr.d, T_MIN, sr.t_max, &tt, &uu, &vv, &tri2,
+                                                           &inst2, &visits, &tests, &overflow);
+                    else
+                        blocked = traverse<true>(sc, st, 0, sr.o, sr.d, T_MIN, sr.t_max, &tt, &uu, &vv, &tri2, &visits,
+                                                 &tests, &overflow);
+                }
+                if (!blocked) P.radiance = v3(P.radiance.x + sr.c.x, P.radiance.y + sr.c.y, P.radiance.z + sr.c.z);
+            }
+            if (!alive) break;
+        }
+        // what RESOLVE reads
+        p.rad[i] = make_float4(P.radiance.x, P.radiance.y, P.radiance.z, 0.0f);
+        p.gal[i] = gal;
+        p.gnr[i] = gnr;
+    }
+    // ray counts into bounce 0's slots (the fold sums every bounce's slot)
+    const uint64_t wr = wave_sum_u32(rays), ws = wave_sum_u32(shadow_rays);
+    if ((threadIdx.x & 63) == 0) {
+        if (wr) atomicAdd(&p.counters[0], (uint32_t)wr);
+        if (ws) atomicAdd(&p.counters[SHADOW_AT], (uint32_t)ws);
+    }
+    flush_traversal_stats(p.counters, 0u, 0u, overflow, 0u, 0);
+}
+
+// ---------------------------------------------------------------------------
 // RESOLVE (resolve.wgsl:305-338): per pixel, sum the batch's samples in sample
 // order and add them to the film.
 // ---------------------------------------------------------------------------
@@ -1904,6 +2006,12 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
     const uint32_t stats_on = (stats && cfg.count_traversal) ? 1u : 0u;
     const bool profile = stats && cfg.profile_kernels;
 
+    // Renders of few paths trace each path in one launch (k_paths), unless the
+    // caller asks for per-stage times, traversal counts, stages alone or sorted
+    // queues.
+    const bool whole_paths = item_paths <= (size_t)ctx->cu_count * PATHS_WAVES_PER_CU * 64 && !stats_on && !profile &&
+                             !cfg.serialize && !sort_rays;
+
     // Optional per-kernel events: one start/stop pair per launch, destroyed
     // on every return path.
     struct EventSet {
@@ -1951,14 +2059,20 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
         LUCIDA_HIP(hipMemcpyAsync(dU, &u, sizeof u, hipMemcpyHostToDevice, s), LUCIDA_VALIDATION);
         hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, s, p.counters, (uint32_t)TOTALS_AT);
         mark(0, true, s);
-        hipLaunchKernelGGL(k_generate, dim3(grid_for(Pb, 256)), dim3(256), 0, s, dU, p, it.band);
+        const dim3 path_grid(grid_for(Pb, TRACE_WG));
+        if (whole_paths && mode == TRAV_INSTANCED)
+            hipLaunchKernelGGL(k_paths<TRAV_INSTANCED>, path_grid, dim3(TRACE_WG), 0, s, sc, dU, p, it.band);
+        else if (whole_paths)
+            hipLaunchKernelGGL(k_paths<TRAV_BINARY>, path_grid, dim3(TRACE_WG), 0, s, sc, dU, p, it.band);
+        else
+            hipLaunchKernelGGL(k_generate, dim3(grid_for(Pb, 256)), dim3(256), 0, s, dU, p, it.band);
         mark(0, false, s);
         // CONNECT of bounce b runs on the second stream beside EXTEND of
         // bounce b + 1 (shadow planes and radiance against queues, rays and
         // hits); SHADE of bounce b + 1 and RESOLVE wait for it (radiance, and
         // the shadow planes SHADE rewrites).
         uint32_t* qin = p.q0;  // GENERATE's queue
-        for (uint32_t b = 0; b < depth; ++b) {
+        for (uint32_t b = 0; b < depth && !whole_paths; ++b) {
             uint32_t* qout = qin == p.q1 ? p.q0 : p.q1;  // SHADE's appends: any queue but the one it reads
             uint32_t* qnext = qout;
             uint32_t* order = nullptr;
@@ -1988,7 +2102,7 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
             LUCIDA_HIP(hipEventRecord(w.ev_connected, s2), LUCIDA_VALIDATION);
             qin = qnext;
         }
-        LUCIDA_HIP(hipStreamWaitEvent(s, w.ev_connected, 0), LUCIDA_VALIDATION);
+        if (!whole_paths) LUCIDA_HIP(hipStreamWaitEvent(s, w.ev_connected, 0), LUCIDA_VALIDATION);
         // batches add into the film in order, whichever pipeline ran them
         if (batch > 0) LUCIDA_HIP(hipStreamWaitEvent(s, ctx->ev_resolved, 0), LUCIDA_VALIDATION);
         mark(4, true, s);
