@@ -135,6 +135,7 @@ void lucida_ctx_destroy(lucida_ctx* ctx) {
     for (WfPipe& w : ctx->wf) {
         DevBuf* wb[] = {&w.planes, &w.hits, &w.shadow, &w.queues, &w.counters, &w.uniforms, &w.spill};
         for (DevBuf* b : wb) b->release();
+        if (w.host_totals) (void)hipHostFree(w.host_totals);
         hipEvent_t evs[] = {w.ev_shaded, w.ev_connected, w.ev_sorted, w.ev_shadow_sorted};
         for (hipEvent_t e : evs)
             if (e) (void)hipEventDestroy(e);

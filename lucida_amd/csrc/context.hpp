@@ -80,6 +80,7 @@ struct WfPipe {
     // the two queue sorts, one per stream, joined before the walks start
     hipEvent_t ev_sorted = nullptr, ev_shadow_sorted = nullptr;
     DevBuf planes, hits, shadow, queues, counters, uniforms, spill;
+    uint64_t* host_totals = nullptr;  // a render's ray and visit totals, in pinned host memory
     size_t capacity = 0;
 };
 

@@ -1582,23 +1582,36 @@ __global__ __launch_bounds__(256) void k_resolve_batch(const BatchJob* __restric
 
 // Adds one batch's counters into the render's running totals (u64 at word
 // TOTALS_AT): extension rays, shadow rays, closest-hit visits and tests,
-// any-hit visits and tests, stack overflows.
-__global__ void k_fold_counters(uint32_t* counters, uint32_t depth) {
-    if (threadIdx.x != 0) return;
+// any-hit visits and tests, stack overflows and the walks' lane slots. One
+// wave: lanes take the bounces, then the stripes, and add up by shuffles (one
+// lane alone took 7 us, one load after another). With `host` (pinned memory)
+// the totals so far are also left there for the host to read.
+__global__ void k_fold_counters(uint32_t* counters, uint32_t depth, uint64_t* host) {
+    static_assert(STATS_STRIPES <= 64 && MAX_BOUNCES <= 64, "a lane per stripe and per bounce");
+    const uint32_t lane = threadIdx.x;
     uint64_t* tot = reinterpret_cast<uint64_t*>(counters + TOTALS_AT);
     const uint64_t* batch = reinterpret_cast<const uint64_t*>(counters + STATS_AT);
-    uint64_t ext = 0, sh = 0;
-    for (uint32_t b = 0; b < depth; ++b) {
-        ext += counters[b];
-        sh += counters[SHADOW_AT + b];
+    uint64_t v[9];
+    v[0] = lane < depth ? counters[lane] : 0u;
+    v[1] = lane < depth ? counters[SHADOW_AT + lane] : 0u;
+    for (int k = 0; k < 7; ++k) v[2 + k] = lane < STATS_STRIPES ? batch[8 * lane + k] : 0u;
+    for (int k = 0; k < 9; ++k) {
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+        if (lane == (uint32_t)k) {
+            const uint64_t t = tot[k] + v[k];
+            tot[k] = t;
+            if (host) host[k] = t;
+        }
     }
-    tot[0] += ext;
-    tot[1] += sh;
-    for (int k = 0; k < 7; ++k) {
-        uint64_t v = 0;
-        for (uint32_t c = 0; c < STATS_STRIPES; ++c) v += batch[8 * c + k];
-        tot[2 + k] += v;
-    }
+}
+
+// Starts a batch: its uniforms, from the launch's arguments, and its cleared
+// counters (n words; the totals too for a pipeline's first batch), in place of
+// a copy from host memory and two launches.
+__global__ void k_begin_batch(GpuUniforms u, GpuUniforms* __restrict__ out, uint32_t* __restrict__ counters,
+                              uint32_t n) {
+    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) counters[k] = 0;
+    if (threadIdx.x == 0) *out = u;
 }
 
 // Clears the per-bounce counters with a kernel (not a memset) so the batch can
@@ -1798,6 +1811,9 @@ static lucida_status ensure_wavefront(WfPipe& w, size_t P, Planes* out, GpuUnifo
     }
     LUCIDA_HIP(w.counters.ensure(COUNTER_BYTES), LUCIDA_OOM);
     LUCIDA_HIP(w.uniforms.ensure(sizeof(GpuUniforms) * 2), LUCIDA_OOM);
+    if (!w.host_totals)
+        LUCIDA_HIP(hipHostMalloc(reinterpret_cast<void**>(&w.host_totals), 16 * sizeof(uint64_t), hipHostMallocDefault),
+                   LUCIDA_OOM);
     const size_t C = w.capacity;
     set_layout(w, out, records);
     uint32_t* q = w.queues.as<uint32_t>();
@@ -2040,24 +2056,19 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
     LUCIDA_HIP(hipEventRecord(ctx->ev0, s0), LUCIDA_VALIDATION);
     for (int q = 0; q < npipes; ++q) {
         if (q > 0) LUCIDA_HIP(hipStreamWaitEvent(ctx->wf[q].s, ctx->ev0, 0), LUCIDA_VALIDATION);
-        hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, ctx->wf[q].s, pl[q].counters,
-                           (uint32_t)TOTALS_AT + 24u);
     }
-    // each batch's uniforms, kept until the render has finished (their
-    // uploads are asynchronous)
-    std::vector<GpuUniforms> host_u(batches, *uniforms);
     for (uint32_t batch = 0; batch < batches; ++batch) {
         const Item& it = items[batch];
         WfPipe& w = ctx->wf[batch % npipes];
         const Planes& p = pl[batch % npipes];
         GpuUniforms* dU = dUs[batch % npipes];
         hipStream_t s = w.s, s2 = cfg.serialize ? w.s : w.s2;
-        GpuUniforms& u = host_u[batch];
+        GpuUniforms u = *uniforms;
         u.sample_offset = uniforms->sample_offset + it.done;
         u.samples_per_launch = it.spb;
         const size_t Pb = (size_t)it.band.count * it.spb;
-        LUCIDA_HIP(hipMemcpyAsync(dU, &u, sizeof u, hipMemcpyHostToDevice, s), LUCIDA_VALIDATION);
-        hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, s, p.counters, (uint32_t)TOTALS_AT);
+        hipLaunchKernelGGL(k_begin_batch, dim3(1), dim3(256), 0, s, u, dU, p.counters,
+                           (uint32_t)TOTALS_AT + (batch < (uint32_t)npipes ? 24u : 0u));
         mark(0, true, s);
         const dim3 path_grid(grid_for(Pb, TRACE_WG));
         if (whole_paths && mode == TRAV_INSTANCED)
@@ -2110,7 +2121,7 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
                            it.band);
         mark(4, false, s);
         LUCIDA_HIP(hipEventRecord(ctx->ev_resolved, s), LUCIDA_VALIDATION);
-        hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, p.counters, depth);
+        hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, p.counters, depth, w.host_totals);
         LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
     }
     for (int q = 1; q < npipes; ++q) {  // join the other pipeline
@@ -2121,12 +2132,9 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
     LUCIDA_HIP(hipEventSynchronize(ctx->ev1), LUCIDA_VALIDATION);
     LUCIDA_HIP(hipGetLastError(), LUCIDA_VALIDATION);
     if (stats) {
-        uint64_t totals[10] = {};
-        for (int q = 0; q < npipes; ++q) {
-            uint64_t t[10];
-            LUCIDA_HIP(hipMemcpy(t, pl[q].counters + TOTALS_AT, sizeof t, hipMemcpyDeviceToHost), LUCIDA_READBACK);
-            for (int k = 0; k < 10; ++k) totals[k] += t[k];
-        }
+        uint64_t totals[9] = {};  // left in pinned memory by the last k_fold_counters
+        for (int q = 0; q < npipes; ++q)
+            for (int k = 0; k < 9; ++k) totals[k] += ctx->wf[q].host_totals[k];
         float ms = 0.0f;
         LUCIDA_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1), LUCIDA_VALIDATION);
         stats->extension_rays = totals[0];
@@ -2208,7 +2216,7 @@ lucida_status lucida_render_megakernel(lucida_ctx* ctx, const lucida_scene* scen
         else
             hipLaunchKernelGGL(k_megakernel<TRAV_BINARY>, grid, block, 0, s, sc, dU + b, film->accum, whole,
                                ctx->mk_spill.as<uint32_t>(), counters, stats_on);
-        hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, counters, 1u);
+        hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, counters, 1u, nullptr);
         LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
     }
     LUCIDA_HIP(hipEventRecord(ctx->ev1, s), LUCIDA_VALIDATION);
@@ -2482,7 +2490,7 @@ lucida_status lucida_render_batch(lucida_ctx* ctx, const lucida_job* jobs, size_
                 hipLaunchKernelGGL(k_resolve, dim3(grid_for(r.pixels, 256)), dim3(256), 0, s, uj, p,
                                    table[r.first].film, whole);
                 if (npipes > 1) chk(hipEventRecord(ctx->ev_resolved, s));
-                hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, p.counters, r.depth);
+                hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, p.counters, r.depth, nullptr);
                 hipLaunchKernelGGL(k_stamp, dim3(1), dim3(64), 0, s, stamps, (uint32_t)(ri + 1));
                 chk(hipGetLastError());
                 continue;
@@ -2514,7 +2522,7 @@ lucida_status lucida_render_batch(lucida_ctx* ctx, const lucida_job* jobs, size_
             hipLaunchKernelGGL(k_resolve_batch, dim3(grid_for(r.pixels, 256)), dim3(256), 0, s, jr, nj,
                                (uint32_t)r.pixels, p);
             if (npipes > 1) chk(hipEventRecord(ctx->ev_resolved, s));
-            hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, p.counters, r.depth);
+            hipLaunchKernelGGL(k_fold_counters, dim3(1), dim3(64), 0, s, p.counters, r.depth, nullptr);
             hipLaunchKernelGGL(k_stamp, dim3(1), dim3(64), 0, s, stamps, (uint32_t)(ri + 1));
             chk(hipGetLastError());
         }
