@@ -130,8 +130,11 @@ void lucida_ctx_destroy(lucida_ctx* ctx) {
                       &ctx->lb_tmpv,   &ctx->lb_hist,    &ctx->lb_karras, &ctx->lb_parent, &ctx->lb_nodebox,
                       &ctx->lb_subtree, &ctx->lb_flags,  &ctx->lb_misc,  &ctx->lb_rank,   &ctx->lb_nodes,
                       &ctx->lb_tris,   &ctx->lb_pos,     &ctx->lb_prims, &ctx->lb_level, &ctx->ggx_table, &ctx->dn_buf,
-                      &ctx->conv_buf, &ctx->mk_spill, &ctx->mk_state};
+                      &ctx->conv_buf, &ctx->mk_spill, &ctx->mk_state,  &ctx->tl_cost,   &ctx->tl_leafy,
+                      &ctx->tl_order,  &ctx->tl_list};
     for (DevBuf* b : bufs) b->release();
+    if (ctx->tl_host) (void)hipHostFree(ctx->tl_host);
+    if (ctx->tl_counted) (void)hipEventDestroy(ctx->tl_counted);
     for (WfPipe& w : ctx->wf) {
         DevBuf* wb[] = {&w.planes, &w.hits, &w.shadow, &w.queues, &w.counters, &w.uniforms, &w.spill};
         for (DevBuf* b : wb) b->release();

@@ -101,6 +101,8 @@ struct lucida_ctx {
         lb_nodebox, lb_subtree, lb_flags, lb_misc, lb_rank, lb_nodes, lb_tris, lb_pos, lb_prims, lb_level;
     // Treelet restructuring: per-node costs, leaf choices, the leaf order.
     lucida::DevBuf tl_cost, tl_leafy, tl_order, tl_list;
+    uint32_t* tl_host = nullptr;       // a round's per-level counts, in pinned host memory,
+    hipEvent_t tl_counted = nullptr;   // and when they are there
     int lbvh_fit = 0;  // 0: two-phase fit (block-local, then the top), 1: atomic bottom-up, 2: level-synchronous
     // GGX directional-albedo table (energy compensation), 32 x 32 floats.
     lucida::DevBuf ggx_table;

@@ -43,41 +43,56 @@ constexpr float CT = LUCIDA_TREELET_CT;
 constexpr uint32_t LEAF_BIT = 0x100u;  // in a subset's part word: the subset is kept as one leaf
 static_assert(LEAVES == 7 && MIN_SIZE >= 3, "one wave covers the 127 subsets of 7 leaves, two per lane");
 
-// One wave's working set for one treelet.
+// One wave's working set for one treelet, by subset of its leaves.
 struct TreeletLds {
-    float box[6][SUBSETS];  // per subset: lo xyz, hi xyz
-    float cost[SUBSETS];
-    uint32_t count[SUBSETS];
+    float2 cost[SUBSETS];   // least cost; primitives (as bits)
+    float box[6][SUBSETS];  // lo xyz, hi xyz
+    float area[SUBSETS];
     uint32_t part[SUBSETS];  // left side of the best split | LEAF_BIT
-    uint32_t icnt[SUBSETS];  // internal nodes the layout emits for the subset's best subtree
-    uint32_t leaf[8];        // the treelet's leaves
-    uint32_t inner[8];       // its internal nodes, the root first
-    uint32_t stack_set[8], stack_slot[8];
 };
 
-// The 127 nonempty subsets of 7 leaves ordered by size, then mask; off[m] is
-// where the subsets of m leaves start.
-struct SubsetTable {
-    uint8_t mask[SUBSETS - 1];
-    uint8_t off[LEAVES + 2];
+// What each lane works on in the dynamic program over the 127 subsets of seven
+// leaves. Subsets of m leaves are solved together, 2^LANE_SHIFT[m] lanes to a
+// subset (21 x 1, 35 x 1, 35 x 1, 21 x 2, 7 x 8 and 1 x 64 lanes), each taking
+// every 2^LANE_SHIFT[m]-th of its 2^(m-1) - 1 partitions. A partition is named by
+// its left side, which keeps the subset's lowest leaf; ascending j deposits j's
+// bits on the other leaves, so a lane's partitions ascend. Subset 0: idle.
+constexpr uint32_t LANE_SHIFT[LEAVES + 1] = {0, 0, 0, 0, 0, 1, 3, 6};
+constexpr int lane_parts(int m) { return ((1 << (m - 1)) - 1 + (1 << LANE_SHIFT[m]) - 1) >> LANE_SHIFT[m]; }
+constexpr int part_byte(int m) { return m == 2 ? 0 : part_byte(m - 1) + lane_parts(m - 1); }
+constexpr int SUBSET_BYTE = part_byte(LEAVES) + lane_parts(LEAVES);  // the lane's subsets of 2, 3, ... leaves
+static_assert(SUBSET_BYTE + LEAVES - 1 <= 32, "a lane's program is 32 bytes");
+struct LaneProgram {
+    uint8_t byte[64][32];
 };
 constexpr int popcount7(int v) { return (v & 1) + (v >> 1 & 1) + (v >> 2 & 1) + (v >> 3 & 1) + (v >> 4 & 1) + (v >> 5 & 1) + (v >> 6 & 1); }
-constexpr SubsetTable make_subset_table() {
-    SubsetTable t{};
-    int n = 0;
-    for (int m = 1; m <= LEAVES; ++m) {
-        t.off[m] = (uint8_t)n;
-        for (int v = 1; v < (int)SUBSETS; ++v)
-            if (popcount7(v) == m) t.mask[n++] = (uint8_t)v;
+constexpr LaneProgram make_lane_program() {
+    LaneProgram t{};
+    for (int m = 2; m <= LEAVES; ++m) {
+        int group = 0;
+        for (int v = 1; v < (int)SUBSETS; ++v) {
+            if (popcount7(v) != m) continue;
+            const int low = v & -v;
+            for (int r = 0; r < 1 << LANE_SHIFT[m]; ++r) {
+                const int lane = (group << LANE_SHIFT[m]) + r;
+                t.byte[lane][SUBSET_BYTE + m - 2] = (uint8_t)v;
+                int at = part_byte(m);
+                for (int j = r; j < (1 << (m - 1)) - 1; j += 1 << LANE_SHIFT[m]) {
+                    int side = low, rest = v ^ low;
+                    for (int b = 1; rest; b <<= 1) {  // j's bits on the other leaves, lowest first
+                        const int bit = rest & -rest;
+                        if (j & b) side |= bit;
+                        rest ^= bit;
+                    }
+                    t.byte[lane][at++] = (uint8_t)side;
+                }
+            }
+            ++group;
+        }
     }
-    t.off[LEAVES + 1] = (uint8_t)n;
     return t;
 }
-__constant__ SubsetTable c_subsets = make_subset_table();
-// Lanes that share one subset's partitions, as a shift, per subset size: the
-// subsets of one size and their 2^(m-1) - 1 partitions spread over the wave
-// (21 x 1, 35 x 1, 35 x 1, 21 x 2, 7 x 8 and 1 x 64 lanes).
-constexpr uint32_t GROUP_SHIFT[LEAVES + 1] = {0, 0, 0, 0, 0, 1, 3, 6};
+__constant__ LaneProgram c_program = make_lane_program();
 
 __device__ inline float area(float lx, float ly, float lz, float hx, float hy, float hz) {
     const float dx = hx - lx, dy = hy - ly, dz = hz - lz;
@@ -111,94 +126,119 @@ struct TreeArrays {
 __device__ inline uint32_t size_of(const TreeArrays& t, uint32_t id) { return id >= t.leaf_base ? 1u : t.size[id]; }
 __device__ inline uint32_t inner_of(const TreeArrays& t, uint32_t id) { return id >= t.leaf_base ? 0u : t.inner[id]; }
 
-// The bits of j placed, lowest first, at the set bits of mask.
-__device__ inline uint32_t deposit(uint32_t j, uint32_t mask) {
-    uint32_t out = 0;
-    for (uint32_t b = 1; mask; b <<= 1) {
-        const uint32_t low = mask & (0u - mask);
-        if (j & b) out |= low;
-        mask ^= low;
-    }
-    return out;
-}
-
-// The least-cost subtrees over all subsets of m leaves, from the costs of
-// their proper subsets (already in LDS). A subset's partitions keep its
-// lowest leaf on the left; partition j's left side is that leaf plus the
-// bits of j deposited on the others, so ascending j is ascending mask. The
-// split chosen is the least (cost, imbalance, mask), imbalance being the
-// difference of the two sides' primitive counts, with costs compared to 20
-// mantissa bits (cost_key): among costs equal up to their rounding (boxes
-// that coincide, summed in different orders) the most even split, so ties do
-// not build chains. The lanes sharing a subset take every G-th partition,
-// keep their first least triple, and then agree on the least. A NaN cost is
-// never chosen; with every cost NaN the split is the lowest leaf alone.
 // A cost with its 4 lowest mantissa bits cleared: monotone in the cost
 // (costs are not negative), so comparing keys is a total order.
 __device__ inline float cost_key(float c) { return __uint_as_float(__float_as_uint(c) & 0xFFFFFFF0u); }
 
-__device__ inline void solve_size(TreeletLds& L, uint32_t lane, int m, uint32_t full) {
-    const uint32_t gs = GROUP_SHIFT[m];
-    const uint32_t g = lane >> gs, r = lane & ((1u << gs) - 1u);
-    const uint32_t first = c_subsets.off[m], nsub = c_subsets.off[m + 1] - first;
+// Values of one lane in every lane (the lane uniform).
+__device__ inline uint32_t lane_u(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
+__device__ inline float lane_f(float v, int lane) { return __uint_as_float(lane_u(__float_as_uint(v), lane)); }
+
+template <int CTRL>
+__device__ inline uint32_t dpp_u(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+
+// The best split so far of a subset: least cost key, then least imbalance,
+// then least left side.
+struct Split {
+    float key;
+    uint32_t im, side;
+    __device__ inline void take(bool valid, float k, uint32_t i, uint32_t s) {
+        // no branches: they cost a lone wave more than the comparisons
+        const bool better = valid & ((k < key) | ((k == key) & ((i < im) | ((i == im) & (s < side)))));
+        key = better ? k : key;
+        im = better ? i : im;
+        side = better ? s : side;
+    }
+    template <int CTRL>
+    __device__ inline void with_dpp() {
+        take(true, __uint_as_float(dpp_u<CTRL>(__float_as_uint(key))), dpp_u<CTRL>(im), dpp_u<CTRL>(side));
+    }
+};
+
+// The least-cost subtrees over all subsets of M leaves, from the costs of
+// their proper subsets (already in LDS). The split chosen is the least (cost,
+// imbalance, mask), imbalance being the difference of the two sides' primitive
+// counts, with costs compared to 20 mantissa bits (cost_key): among costs
+// equal up to their rounding (boxes that coincide, summed in different
+// orders) the most even split, so ties do not build chains. A NaN cost is
+// never chosen; with every cost NaN the split is the lowest leaf alone.
+template <int M>
+__device__ inline void solve_size(TreeletLds& L, uint32_t lane, const uint32_t (&prog)[8], uint32_t full) {
+    auto byte = [&](int k) { return (prog[k >> 2] >> (8 * (k & 3))) & 0xFFu; };
+    constexpr int N = lane_parts(M);
+    uint32_t s = byte(SUBSET_BYTE + M - 2);
+    if (s > full) s = 0;
     const float inf = __builtin_huge_valf();
-    float key = inf;
-    uint32_t bp = 0xFFu, bim = 0xFFFFFFFFu, s = 0;
-    if (g < nsub) {
-        s = c_subsets.mask[first + g];
-        if (s <= full) {
-            const uint32_t low = s & (0u - s), rest = s ^ low;
-            const uint32_t parts = (1u << (m - 1)) - 1u;
-            for (uint32_t j = r; j < parts; j += 1u << gs) {
-                const uint32_t pm = low | deposit(j, rest);
-                const float cand = L.cost[pm] + L.cost[s ^ pm];
-                if (!(cand == cand)) continue;  // NaN
-                const float qc = cost_key(cand);
-                if (qc <= key) {  // the counts are read only for a lower or equal key
-                    const uint32_t np = L.count[pm], nq = L.count[s ^ pm];
-                    const uint32_t im = np > nq ? np - nq : nq - np;
-                    if (qc < key || im < bim) {
-                        key = qc;
-                        bim = im;
-                        bp = pm;
-                    }
-                }
-            }
-        }
+    Split best{inf, 0xFFFFFFFFu, 0xFFu};
+    const float count_bits = L.cost[s].y;
+    const uint32_t count = __float_as_uint(count_bits);
+    const float a = L.area[s];
+    float2 left[N];
+    float right[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {  // side 0 (no partition, or an idle lane): subset 0, not looked at
+        const uint32_t side = s ? byte(part_byte(M) + j) : 0u;
+        left[j] = L.cost[side];
+        right[j] = L.cost[s ^ side].x;
     }
-    for (uint32_t o = 1; o < (1u << gs); o <<= 1) {
-        const float ok = __shfl_xor(key, o, 64);
-        const uint32_t oi = __shfl_xor(bim, o, 64);
-        const uint32_t op = __shfl_xor(bp, o, 64);
-        if (ok < key || (ok == key && (oi < bim || (oi == bim && op < bp)))) {
-            key = ok;
-            bim = oi;
-            bp = op;
-        }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const uint32_t side = s ? byte(part_byte(M) + j) : 0u;
+        const float cand = left[j].x + right[j];
+        const uint32_t np = __float_as_uint(left[j].y), nq = count - np;
+        best.take((side != 0) & (cand == cand), cost_key(cand), np > nq ? np - nq : nq - np, side);
     }
-    if (r == 0 && g < nsub && s <= full) {
-        float best = inf;
-        if (bp == 0xFFu)
-            bp = s & (0u - s);
+    if (LANE_SHIFT[M] >= 1) best.with_dpp<0xB1>();   // lane ^ 1
+    if (LANE_SHIFT[M] >= 2) best.with_dpp<0x4E>();   // lane ^ 2
+    if (LANE_SHIFT[M] >= 3) best.with_dpp<0x141>();  // the other half of eight lanes
+    if (LANE_SHIFT[M] >= 6) {
+        best.with_dpp<0x140>();  // the other half of sixteen
+        Split all{lane_f(best.key, 0), lane_u(best.im, 0), lane_u(best.side, 0)};
+        for (int row = 16; row < 64; row += 16) all.take(true, lane_f(best.key, row), lane_u(best.im, row), lane_u(best.side, row));
+        best = all;
+    }
+    if (s && (lane & ((1u << LANE_SHIFT[M]) - 1u)) == 0) {
+        uint32_t side = best.side;
+        float split = inf;
+        if (side == 0xFFu)
+            side = s & (0u - s);
         else
-            best = L.cost[bp] + L.cost[s ^ bp];
-        const float a = area(L.box[0][s], L.box[1][s], L.box[2][s], L.box[3][s], L.box[4][s], L.box[5][s]);
-        const float inner = CI * a + best;
-        const float leaf = CT * a * (float)L.count[s];
-        const bool as_leaf = L.count[s] <= MAX_LEAF && leaf <= inner;
-        L.cost[s] = as_leaf ? leaf : inner;
-        L.part[s] = bp | (as_leaf ? LEAF_BIT : 0u);
-        L.icnt[s] = as_leaf ? 0u : 1u + L.icnt[bp] + L.icnt[s ^ bp];
+            split = L.cost[side].x + L.cost[s ^ side].x;
+        const float inner = CI * a + split;
+        const float leaf = CT * a * (float)count;
+        const bool as_leaf = count <= MAX_LEAF && leaf <= inner;
+        L.cost[s] = make_float2(as_leaf ? leaf : inner, count_bits);
+        L.part[s] = side | (as_leaf ? LEAF_BIT : 0u);
     }
 }
 
 // The whole wave rebuilds the treelet under node x (uniform).
+//
+// What bounds it is the latency of one treelet, as the levels follow each
+// other and most hold fewer treelets than the device has wave slots: dependent
+// loads, then chains of cross-lane and LDS steps. So every node the treelet may
+// take is fetched with all its data in one round of loads, values travel
+// between lanes through readlane and DPP rather than LDS, a lane's partitions
+// come from a table and are all read before any is compared, and the rebuilt
+// nodes are written by a lane each. A level of few treelets takes 14 us (19
+// with LDS permutes, bit deposits and one lane rebuilding), the largest of the
+// 328,704-triangle mesh (14,880 treelets) 53 us, where the instructions
+// themselves bound it; three rounds there 2,655 -> 1,640 us. One workgroup
+// walking the top levels without launches took as long a level, 13 us.
 __device__ void restructure(const TreeArrays& t, TreeletLds& L, uint32_t lane, uint32_t x) {
-    wave_sync();  // the previous treelet's LDS reads are done
+    uint32_t prog[8];
+    {
+        const uint4* q = reinterpret_cast<const uint4*>(c_program.byte[lane]);
+        const uint4 a = q[0], b = q[1];
+        prog[0] = a.x; prog[1] = a.y; prog[2] = a.z; prog[3] = a.w;
+        prog[4] = b.x; prog[5] = b.y; prog[6] = b.z; prog[7] = b.w;
+    }
     // The three levels under x, fetched across lanes first: heap slot p < 14
-    // (lane p) holds a node id and its area (-1 for a primitive, which is
-    // never opened); slots 0 and 1 are x's children and slot p >= 2 is child
-    // p & 1 of slot (p - 2) / 2.
+    // (lane p) holds a node; slots 0 and 1 are x's children and slot p >= 2 is
+    // child p & 1 of slot (p - 2) / 2. Slots 14 on are taken in pairs for the
+    // children of deeper nodes.
     const uint2 c0 = t.child[x];
     uint32_t hid = lane == 0 ? c0.x : (lane == 1 ? c0.y : NONE);
     for (uint32_t lo = 2, hi = 6; lo < 14; lo = hi, hi = 2 * hi + 2) {
@@ -208,167 +248,203 @@ __device__ void restructure(const TreeArrays& t, TreeletLds& L, uint32_t lane, u
             hid = (lane & 1u) ? c.y : c.x;
         }
     }
-    const bool hin = lane < 14 && hid < t.leaf_base;
-    const float harea = hin ? node_area(t.box, hid) : -1.0f;
-    const uint32_t hsize = hin ? t.size[hid] : 0u;
-    // Grow: lane i < k holds leaf i (id, area, primitives, heap slot or NONE);
-    // the leaf of largest area, then most primitives (the first such), is
-    // replaced by its left child and its right child appended.
-    uint32_t id = __shfl(hid, lane < 2 ? lane : 0u, 64);
-    float id_area = __shfl(harea, lane < 2 ? lane : 0u, 64);
-    uint32_t id_size = __shfl(hsize, lane < 2 ? lane : 0u, 64);
-    uint32_t hpos = lane;
-    if (lane >= 2) {
-        id = NONE;
-        id_area = -1.0f;
-        id_size = 0;
-        hpos = NONE;
-    }
+    // A slot's node: its box, cost, size and emitted-internal count; the area is
+    // -1 for a primitive, which is never opened.
+    float4 blo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), bhi = blo;
+    float harea = -1.0f, hcost = 0.0f;
+    uint32_t hsize = 0, hinner = 0;
+    auto fetch = [&]() {
+        const float4* p = reinterpret_cast<const float4*>(t.box + hid);
+        blo = p[0];
+        bhi = p[1];
+        hcost = t.cost[hid];
+        hsize = size_of(t, hid);
+        hinner = inner_of(t, hid);
+        harea = hid < t.leaf_base ? area(blo.x, blo.y, blo.z, bhi.x, bhi.y, bhi.z) : -1.0f;
+    };
+    if (hid != NONE) fetch();
+    // Grow: lane i < k holds leaf i's slot, area and primitives (0 for one
+    // that is a primitive itself); the leaf of largest area, then most
+    // primitives (the first such), is replaced by its left child and its
+    // right child appended.
+    uint32_t slot = lane < 2 ? lane : 0u;
+    float leaf_area = lane < 2 ? harea : -1.0f;
+    uint32_t leaf_size = lane < 2 && hid < t.leaf_base ? hsize : 0u;
     uint32_t inner_id = lane == 0 ? x : NONE;
-    int k = 2;
+    int k = 2, used = 14;
     while (k < LEAVES) {
         int best = -1;
         float best_a = -1.0f;
         uint32_t best_n = 0;
         for (int i = 0; i < k; ++i) {
-            const float a = __shfl(id_area, i, 64);
-            const uint32_t sz = __shfl(id_size, i, 64);
-            if (a >= 0.0f && (a > best_a || (a == best_a && sz > best_n))) {
-                best_a = a;
-                best_n = sz;
-                best = i;
-            }
+            const float a = lane_f(leaf_area, i);
+            const uint32_t sz = lane_u(leaf_size, i);
+            const bool better = (a >= 0.0f) & ((a > best_a) | ((a == best_a) & (sz > best_n)));
+            best_a = better ? a : best_a;
+            best_n = better ? sz : best_n;
+            best = better ? i : best;
         }
+        best = __builtin_amdgcn_readfirstlane(best);
         if (best < 0) break;
-        const uint32_t e = __shfl(id, best, 64);
-        const uint32_t ep = __shfl(hpos, best, 64);
-        uint32_t cx, cy, px = NONE, py = NONE, nx, ny;
-        float ax, ay;
+        const int ep = (int)lane_u(slot, best);
+        const uint32_t e = lane_u(hid, ep);
+        int px;
         if (ep < 6) {  // its children are in the heap
             px = 2 * ep + 2;
-            py = px + 1;
-            cx = __shfl(hid, px, 64);
-            cy = __shfl(hid, py, 64);
-            ax = __shfl(harea, px, 64);
-            ay = __shfl(harea, py, 64);
-            nx = __shfl(hsize, px, 64);
-            ny = __shfl(hsize, py, 64);
         } else {
-            const uint2 ce = t.child[e];
-            cx = ce.x;
-            cy = ce.y;
-            ax = cx < t.leaf_base ? node_area(t.box, cx) : -1.0f;
-            ay = cy < t.leaf_base ? node_area(t.box, cy) : -1.0f;
-            nx = cx < t.leaf_base ? t.size[cx] : 0u;
-            ny = cy < t.leaf_base ? t.size[cy] : 0u;
+            px = used;
+            used += 2;
+            if ((int)lane == px || (int)lane == px + 1) {
+                const uint2 ce = t.child[e];
+                hid = (int)lane == px ? ce.x : ce.y;
+                fetch();
+            }
         }
+        const uint32_t cx = lane_u(hid, px), cy = lane_u(hid, px + 1);
+        const float ax = lane_f(harea, px), ay = lane_f(harea, px + 1);
+        const uint32_t nx = cx < t.leaf_base ? lane_u(hsize, px) : 0u, ny = cy < t.leaf_base ? lane_u(hsize, px + 1) : 0u;
         if (lane == (uint32_t)(k - 1)) inner_id = e;
         if (lane == (uint32_t)best) {
-            id = cx;
-            id_area = ax;
-            id_size = nx;
-            hpos = px;
+            slot = (uint32_t)px;
+            leaf_area = ax;
+            leaf_size = nx;
         }
         if (lane == (uint32_t)k) {
-            id = cy;
-            id_area = ay;
-            id_size = ny;
-            hpos = py;
+            slot = (uint32_t)px + 1;
+            leaf_area = ay;
+            leaf_size = ny;
         }
         ++k;
     }
-    // The leaves' boxes, costs and sizes.
-    float lo0 = 0, lo1 = 0, lo2 = 0, hi0 = 0, hi1 = 0, hi2 = 0, my_cost = 0;
-    uint32_t my_size = 0;
-    if (lane < (uint32_t)k) {
-        const float4* p = reinterpret_cast<const float4*>(t.box + id);
-        const float4 a = p[0], b = p[1];
-        lo0 = a.x; lo1 = a.y; lo2 = a.z;
-        hi0 = b.x; hi1 = b.y; hi2 = b.z;
-        my_cost = t.cost[id];
-        my_size = size_of(t, id);
-        L.leaf[lane] = id;
-        L.icnt[1u << lane] = inner_of(t, id);
-    }
-    if (lane < (uint32_t)(k - 1)) L.inner[lane] = inner_id;
     // Subset boxes and counts: lane l covers subsets l + 1 and l + 65; each
-    // box is the union of its leaves in ascending leaf order.
+    // box is the union of its leaves in ascending leaf order (l + 65 has those
+    // of l + 1, then leaf 6).
     const uint32_t full = (1u << k) - 1;
     const uint32_t s0 = lane + 1, s1 = lane + 65;
     const float inf = __builtin_huge_valf();
-    float a0[6] = {inf, inf, inf, -inf, -inf, -inf}, a1[6] = {inf, inf, inf, -inf, -inf, -inf};
+    float lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf}, lo1[3], hi1[3];
     uint32_t n0 = 0, n1 = 0;
+    uint32_t leaf_id = NONE, leaf_inner = 0;  // leaf `lane`'s
+    float my_cost = 0.0f;
     for (int i = 0; i < k; ++i) {
-        const float q[6] = {__shfl(lo0, i, 64), __shfl(lo1, i, 64), __shfl(lo2, i, 64),
-                            __shfl(hi0, i, 64), __shfl(hi1, i, 64), __shfl(hi2, i, 64)};
-        const uint32_t qs = __shfl(my_size, i, 64);
-        if (s0 >> i & 1u) {
+        const int sl = (int)lane_u(slot, i);
+        const bool in0 = s0 >> i & 1u;
+        const float ql[3] = {lane_f(blo.x, sl), lane_f(blo.y, sl), lane_f(blo.z, sl)};
+        const float qh[3] = {lane_f(bhi.x, sl), lane_f(bhi.y, sl), lane_f(bhi.z, sl)};
+        const uint32_t qs = lane_u(hsize, sl);
+        if (i == LEAVES - 1) {
             for (int j = 0; j < 3; ++j) {
-                a0[j] = fminf(a0[j], q[j]);
-                a0[j + 3] = fmaxf(a0[j + 3], q[j + 3]);
+                lo1[j] = fminf(lo[j], ql[j]);
+                hi1[j] = fmaxf(hi[j], qh[j]);
             }
-            n0 += qs;
+            n1 = n0 + qs;
         }
-        if (s1 >> i & 1u) {
-            for (int j = 0; j < 3; ++j) {
-                a1[j] = fminf(a1[j], q[j]);
-                a1[j + 3] = fmaxf(a1[j + 3], q[j + 3]);
-            }
-            n1 += qs;
+        for (int j = 0; j < 3; ++j) {
+            lo[j] = fminf(lo[j], in0 ? ql[j] : inf);
+            hi[j] = fmaxf(hi[j], in0 ? qh[j] : -inf);
         }
+        n0 += in0 ? qs : 0u;
+        if ((int)lane == i) {
+            leaf_id = lane_u(hid, sl);
+            leaf_inner = lane_u(hinner, sl);
+        }
+        const float qc = lane_f(hcost, sl);
+        if (s0 == 1u << i) my_cost = qc;
     }
+    wave_sync();  // the previous treelet's LDS reads are done
     if (s0 <= full) {
-        for (int j = 0; j < 6; ++j) L.box[j][s0] = a0[j];
-        L.count[s0] = n0;
+        for (int j = 0; j < 3; ++j) {
+            L.box[j][s0] = lo[j];
+            L.box[j + 3][s0] = hi[j];
+        }
+        L.area[s0] = area(lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]);
+        L.cost[s0] = make_float2(my_cost, __uint_as_float(n0));
     }
     if (s1 <= full) {
-        for (int j = 0; j < 6; ++j) L.box[j][s1] = a1[j];
-        L.count[s1] = n1;
-    }
-    if (lane < (uint32_t)k) {
-        L.cost[1u << lane] = my_cost;
-        L.part[1u << lane] = 0;
+        for (int j = 0; j < 3; ++j) {
+            L.box[j][s1] = lo1[j];
+            L.box[j + 3][s1] = hi1[j];
+        }
+        L.area[s1] = area(lo1[0], lo1[1], lo1[2], hi1[0], hi1[1], hi1[2]);
+        L.cost[s1] = make_float2(0.0f, __uint_as_float(n1));
     }
     wave_sync();
     // Least costs, subsets of 2 leaves first, then 3, ...
-    for (int m = 2; m <= k; ++m) {
-        solve_size(L, lane, m, full);
-        wave_sync();
-    }
+    solve_size<2>(L, lane, prog, full);
+    wave_sync();
+    if (k >= 3) solve_size<3>(L, lane, prog, full);
+    wave_sync();
+    if (k >= 4) solve_size<4>(L, lane, prog, full);
+    wave_sync();
+    if (k >= 5) solve_size<5>(L, lane, prog, full);
+    wave_sync();
+    if (k >= 6) solve_size<6>(L, lane, prog, full);
+    wave_sync();
+    if (k >= 7) solve_size<7>(L, lane, prog, full);
+    wave_sync();
     // Rebuild in pre-order, left side first, reusing the treelet's internal
-    // nodes in the order they were taken.
-    if (lane == 0) {
-        uint32_t sp = 1, next = 1;
-        L.stack_set[0] = full;
-        L.stack_slot[0] = x;
-        while (sp) {
-            --sp;
-            const uint32_t s = L.stack_set[sp], slot = L.stack_slot[sp];
-            const uint32_t pw = L.part[s];
-            const uint32_t pm = pw & (SUBSETS - 1), qm = s ^ pm;
-            const uint32_t lc = __popc(pm) == 1 ? L.leaf[__ffs(pm) - 1] : L.inner[next++];
-            const uint32_t rc = __popc(qm) == 1 ? L.leaf[__ffs(qm) - 1] : L.inner[next++];
-            t.child[slot] = make_uint2(lc, rc);
-            t.parent[lc] = slot;
-            t.parent[rc] = slot;
-            float4* bp = reinterpret_cast<float4*>(t.box + slot);
-            bp[0] = make_float4(L.box[0][s], L.box[1][s], L.box[2][s], 0.0f);
-            bp[1] = make_float4(L.box[3][s], L.box[4][s], L.box[5][s], 0.0f);
-            t.size[slot] = L.count[s];
-            t.cost[slot] = L.cost[s];
-            t.leafy[slot] = (pw & LEAF_BIT) ? 1u : 0u;
-            t.inner[slot] = L.icnt[s];
-            if (__popc(qm) > 1) {
-                L.stack_set[sp] = qm;
-                L.stack_slot[sp] = rc;
-                ++sp;
-            }
-            if (__popc(pm) > 1) {
-                L.stack_set[sp] = pm;
-                L.stack_slot[sp] = lc;
-                ++sp;
-            }
+    // nodes in the order they were taken: lane j gets the j-th node's subset,
+    // id, split and children; the stack of subtrees to come is in lanes too.
+    uint32_t st_set = full, st_id = x;  // stack entry `lane`
+    uint32_t my_set = 0, my_id = 0, my_part = 0, my_l = 0, my_r = 0;
+    int sp = 1, next = 1, nodes = 0;
+    while (sp) {
+        --sp;
+        const uint32_t s = lane_u(st_set, sp), id = lane_u(st_id, sp);
+        const uint32_t pw = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.part[s]);
+        const uint32_t pm = pw & (SUBSETS - 1), qm = s ^ pm;
+        const bool lone = __popc(pm) == 1, rone = __popc(qm) == 1;
+        const uint32_t lc = lone ? lane_u(leaf_id, __ffs(pm) - 1) : lane_u(inner_id, next);
+        next += lone ? 0 : 1;
+        const uint32_t rc = rone ? lane_u(leaf_id, __ffs(qm) - 1) : lane_u(inner_id, next);
+        next += rone ? 0 : 1;
+        if ((int)lane == nodes) {
+            my_set = s;
+            my_id = id;
+            my_part = pw;
+            my_l = lc;
+            my_r = rc;
         }
+        ++nodes;
+        if (!rone) {
+            if ((int)lane == sp) {
+                st_set = qm;
+                st_id = rc;
+            }
+            ++sp;
+        }
+        if (!lone) {
+            if ((int)lane == sp) {
+                st_set = pm;
+                st_id = lc;
+            }
+            ++sp;
+        }
+    }
+    // emitted-internal counts, children (later in pre-order) first
+    uint32_t my_inner = 0;
+    for (int j = nodes - 1; j >= 0; --j) {
+        const uint32_t s = lane_u(my_set, j), pw = lane_u(my_part, j);
+        const uint32_t pm = pw & (SUBSETS - 1);
+        auto emitted = [&](uint32_t set) {
+            if (__popc(set) == 1) return lane_u(leaf_inner, __ffs(set) - 1);
+            return lane_u(my_inner, __ffsll((unsigned long long)__ballot(my_set == set)) - 1);
+        };
+        const uint32_t both = 1u + emitted(pm) + emitted(s ^ pm);
+        if ((int)lane == j) my_inner = (pw & LEAF_BIT) ? 0u : both;
+    }
+    if ((int)lane < nodes) {
+        t.child[my_id] = make_uint2(my_l, my_r);
+        t.parent[my_l] = my_id;
+        t.parent[my_r] = my_id;
+        float4* bp = reinterpret_cast<float4*>(t.box + my_id);
+        bp[0] = make_float4(L.box[0][my_set], L.box[1][my_set], L.box[2][my_set], 0.0f);
+        bp[1] = make_float4(L.box[3][my_set], L.box[4][my_set], L.box[5][my_set], 0.0f);
+        const float2 c = L.cost[my_set];
+        t.size[my_id] = __float_as_uint(c.y);
+        t.cost[my_id] = c.x;
+        t.leafy[my_id] = (my_part & LEAF_BIT) ? 1u : 0u;
+        t.inner[my_id] = my_inner;
     }
 }
 
@@ -450,9 +526,10 @@ __global__ __launch_bounds__(TL_BLOCK) void k_tl_level(TreeArrays t, const uint3
                                                        uint32_t count) {
     __shared__ TreeletLds lds[TL_WAVES];
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t w = blockIdx.x * TL_WAVES + threadIdx.x / 64;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
+    const uint32_t w = blockIdx.x * TL_WAVES + wave;
     if (w < waves) {
-        restructure(t, lds[threadIdx.x / 64], lane, big[w]);
+        restructure(t, lds[wave], lane, (uint32_t)__builtin_amdgcn_readfirstlane((int)big[w]));
         return;
     }
     const uint32_t i = (w - waves) * 64 + lane;
@@ -469,15 +546,27 @@ __global__ __launch_bounds__(256) void k_clear_words(uint32_t* __restrict__ p, u
     if (i < count) p[i] = 0u;
 }
 
-// Bucket cursors: the exclusive prefix sum of the per-(level, class) counts
-// (one lane; 256 entries).
-__global__ void k_tl_offsets(const uint32_t* __restrict__ count, uint32_t* __restrict__ cursor) {
-    if (threadIdx.x != 0) return;
-    uint32_t acc = 0;
-    for (uint32_t k = 0; k < 2 * MAX_LEVELS; ++k) {
-        cursor[k] = acc;
-        acc += count[k];
+// Bucket cursors: the exclusive prefix sum of the per-(level, class) counts,
+// one thread a count; the counts, then the fault word, also to pinned host
+// memory, so that the host plans the round's launches while the nodes are
+// bucketed.
+__global__ __launch_bounds__(2 * MAX_LEVELS) void k_tl_offsets(const uint32_t* __restrict__ count,
+                                                               const uint32_t* __restrict__ fault,
+                                                               uint32_t* __restrict__ cursor,
+                                                               uint32_t* __restrict__ host) {
+    __shared__ uint32_t sum[2 * MAX_LEVELS];
+    const uint32_t k = threadIdx.x, own = count[k];
+    sum[k] = own;
+    __syncthreads();
+    for (uint32_t o = 1; o < 2 * MAX_LEVELS; o <<= 1) {
+        const uint32_t before = k >= o ? sum[k - o] : 0u;
+        __syncthreads();
+        sum[k] += before;
+        __syncthreads();
     }
+    cursor[k] = sum[k] - own;
+    host[k] = own;
+    if (k == 0) host[2 * MAX_LEVELS] = *fault;
 }
 
 // Layout: an emitted internal node of pre-order rank R among emitted internal
@@ -589,15 +678,27 @@ lucida_status bvh_build_treelet_device(lucida_ctx* ctx, const GpuTriangle* tris,
     uint32_t* level_count = list + internal;
     uint32_t* cursor = level_count + 2 * MAX_LEVELS;
     uint32_t* key = ctx->lb_flags.as<uint32_t>();  // per internal node: 2 x depth + treelet root
+    if (!ctx->tl_host)
+        LUCIDA_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->tl_host), (2 * MAX_LEVELS + 1) * 4,
+                                 hipHostMallocDefault),
+                   LUCIDA_OOM);
+    if (!ctx->tl_counted)
+        LUCIDA_HIP(hipEventCreateWithFlags(&ctx->tl_counted, hipEventDisableTiming), LUCIDA_VALIDATION);
+    const volatile uint32_t* pinned = ctx->tl_host;
     hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(256), 0, s, fault, 1u);
     hipLaunchKernelGGL(k_tl_leaf_cost, dim3(blocks_for(n, 256)), dim3(256), 0, s, t);
     for (uint32_t r = 0; r < (rounds ? rounds : 1u); ++r) {
         hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(256), 0, s, level_count, 2 * MAX_LEVELS);
         hipLaunchKernelGGL(k_tl_depth, dim3(blocks_for(internal, 256)), dim3(256), 0, s, t, key, level_count, fault);
+        hipLaunchKernelGGL(k_tl_offsets, dim3(1), dim3(2 * MAX_LEVELS), 0, s, level_count, fault, cursor,
+                           ctx->tl_host);
+        LUCIDA_HIP(hipEventRecord(ctx->tl_counted, s), LUCIDA_VALIDATION);
+        hipLaunchKernelGGL(k_tl_bucket, dim3(blocks_for(internal, 256)), dim3(256), 0, s, (uint32_t)internal, key,
+                           cursor, list);
+        LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
+        LUCIDA_HIP(hipEventSynchronize(ctx->tl_counted), LUCIDA_VALIDATION);
         uint32_t host[2 * MAX_LEVELS + 1];
-        LUCIDA_HIP(hipMemcpyAsync(host, level_count, 2 * MAX_LEVELS * 4, hipMemcpyDeviceToHost, s), LUCIDA_READBACK);
-        LUCIDA_HIP(hipMemcpyAsync(host + 2 * MAX_LEVELS, fault, 4, hipMemcpyDeviceToHost, s), LUCIDA_READBACK);
-        LUCIDA_HIP(hipStreamSynchronize(s), LUCIDA_VALIDATION);
+        for (uint32_t k = 0; k <= 2 * MAX_LEVELS; ++k) host[k] = pinned[k];
         if (host[2 * MAX_LEVELS]) return set_error(LUCIDA_VALIDATION, "treelet BVH: deeper than 128 levels");
         uint32_t off[2 * MAX_LEVELS], acc = 0;
         int deepest = 0;
@@ -606,10 +707,6 @@ lucida_status bvh_build_treelet_device(lucida_ctx* ctx, const GpuTriangle* tris,
             acc += host[k];
             if (host[k]) deepest = (int)(k / 2);
         }
-        // the device forms the same offsets as its bucket cursors, in stream order
-        hipLaunchKernelGGL(k_tl_offsets, dim3(1), dim3(64), 0, s, level_count, cursor);
-        hipLaunchKernelGGL(k_tl_bucket, dim3(blocks_for(internal, 256)), dim3(256), 0, s, (uint32_t)internal, key,
-                           cursor, list);
         for (int d = deepest; d >= 0; --d) {
             const uint32_t nsmall = host[2 * d], nbig = host[2 * d + 1];
             if (!nsmall && !nbig) continue;
