@@ -309,7 +309,7 @@ lucida_status lucida_sort_u32_device(lucida_ctx* ctx, uint32_t* keys, uint32_t* 
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): lucida_sort_u32_device with its histogram and scan
- * scratch in a fixed per-GPU array inside the library (8 MiB + 4 KiB, held
+ * scratch in a fixed per-GPU array inside the library (8 MiB + 1 KiB, held
  * until the process ends) instead of the context's growing buffer. It calls
  * no allocator. n may be at most LUCIDA_SORT_NOALLOC_MAX_KEYS (2^24); larger
  * n is LUCIDA_INVALID_ARG. Queued on the context's stream like

@@ -164,9 +164,6 @@ lucida_status bvh_build_treelet_device(lucida_ctx* ctx, const GpuTriangle* tris,
 // (lbvh.hip), once per device; lucida_ctx_create calls it with ctx->device
 // current.
 lucida_status sort_scratch_init(lucida_ctx* ctx);
-// Exclusive prefix sum of device words in place (lbvh.hip); `partials` holds
-// ceil(count / 2048) words.
-lucida_status scan_u32_device(lucida_ctx* ctx, uint32_t* data, uint32_t count, uint32_t* partials);
 // Stable radix sort of (keys, vals)[0, *count) by the low `bits` (a multiple
 // of 8) key bits on `stream` (lbvh.hip); the count is a device word at most
 // `capacity`; tk/tv are temporaries of `capacity` words, `scratch` holds

@@ -188,7 +188,7 @@ __global__ __launch_bounds__(PREP_BLOCK) void k_morton(const LucidaAabb* __restr
 
 // ---------------------------------------------------------------------------
 // LSD radix sort, 8-bit digits. Per pass: per-tile digit histograms (LDS
-// atomics), one exclusive scan over the digit-major histogram, then a stable
+// atomics), an exclusive scan of each digit's row of them, then a stable
 // scatter whose in-tile ranks come from wave64 ballots: eight ballots give
 // every lane the set of lanes holding its digit, a popcount below the lane
 // gives its rank among them, a wave counts its digits in LDS of its own as it
@@ -218,11 +218,6 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_radix_hist(const uint32_t* __res
     hist[threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Exclusive scan of the digit-major histogram, in two launches: per-segment
-// sums (k_scan_reduce), then a scan of each segment from its carry, the sum
-// of the segment sums before it, which each block adds up itself
-// (k_scan_down). Every global access is coalesced; a
-// segment is SCAN_ITEMS words per thread of a SCAN_BLOCK block.
 constexpr int SCAN_BLOCK = 256;
 constexpr int SCAN_ITEMS = 8;
 constexpr int SCAN_SEG = SCAN_BLOCK * SCAN_ITEMS;
@@ -250,57 +245,35 @@ __device__ inline uint32_t block_inclusive_scan(uint32_t v, uint32_t* wsum, uint
     return v + before;
 }
 
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(const uint32_t* __restrict__ data, uint32_t count,
-                                                            uint32_t* __restrict__ partials) {
+// The exclusive scan of one digit's row of a digit-major histogram (blockIdx.x
+// the digit), over the tiles, in place; its total to totals[digit]. The
+// scatter's blocks scan the 256 totals themselves, so a pass takes one launch
+// and one reading of the histogram here, where a scan across all digits took
+// two (3.8 us each at 1.05M keys).
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_rows(uint32_t* __restrict__ hist, uint32_t tiles,
+                                                          uint32_t* __restrict__ totals) {
     __shared__ uint32_t wsum[SCAN_BLOCK / 64];
-    const uint32_t base = blockIdx.x * SCAN_SEG;
-    uint32_t s = 0;
+    uint32_t* row = hist + (size_t)blockIdx.x * tiles;
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < tiles; base += SCAN_SEG) {
+        // thread t owns words [base + t * SCAN_ITEMS, + SCAN_ITEMS)
+        uint32_t v[SCAN_ITEMS], s = 0;
+        const uint32_t at = base + threadIdx.x * SCAN_ITEMS;
 #pragma unroll
-    for (int r = 0; r < SCAN_ITEMS; ++r) {
-        const uint32_t idx = base + r * SCAN_BLOCK + threadIdx.x;
-        if (idx < count) s += data[idx];
-    }
-    uint32_t total;
-    (void)block_inclusive_scan(s, wsum, &total);
-    if (threadIdx.x == 0) partials[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(uint32_t* __restrict__ data, uint32_t count,
-                                                          const uint32_t* __restrict__ partials) {
-    __shared__ uint32_t seg[SCAN_SEG];
-    __shared__ uint32_t wsum[SCAN_BLOCK / 64];
-    const uint32_t base = blockIdx.x * SCAN_SEG;
+        for (int i = 0; i < SCAN_ITEMS; ++i) {
+            v[i] = at + i < tiles ? row[at + i] : 0u;
+            s += v[i];
+        }
+        uint32_t total;
+        uint32_t run = carry + block_inclusive_scan(s, wsum, &total) - s;
 #pragma unroll
-    for (int r = 0; r < SCAN_ITEMS; ++r) {
-        const uint32_t idx = base + r * SCAN_BLOCK + threadIdx.x;
-        seg[r * SCAN_BLOCK + threadIdx.x] = idx < count ? data[idx] : 0u;
+        for (int i = 0; i < SCAN_ITEMS; ++i) {
+            if (at + i < tiles) row[at + i] = run;
+            run += v[i];
+        }
+        carry += total;
     }
-    __syncthreads();
-    // thread t owns segment words [t * SCAN_ITEMS, (t + 1) * SCAN_ITEMS)
-    uint32_t local[SCAN_ITEMS];
-    uint32_t s = 0;
-#pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; ++i) {
-        local[i] = seg[threadIdx.x * SCAN_ITEMS + i];
-        s += local[i];
-    }
-    // this segment's carry: the sums of the segments before it
-    uint32_t before = 0;
-    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += SCAN_BLOCK) before += partials[b];
-    uint32_t carry, total;
-    (void)block_inclusive_scan(before, wsum, &carry);
-    uint32_t run = carry + block_inclusive_scan(s, wsum, &total) - s;
-#pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; ++i) {
-        seg[threadIdx.x * SCAN_ITEMS + i] = run;
-        run += local[i];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < SCAN_ITEMS; ++r) {
-        const uint32_t idx = base + r * SCAN_BLOCK + threadIdx.x;
-        if (idx < count) data[idx] = seg[r * SCAN_BLOCK + threadIdx.x];
-    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
 
 // The scatter stages its tile in LDS: items are ranked within the tile by
@@ -317,7 +290,8 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(uint32_t* __restrict__
 __global__ __launch_bounds__(SORT_BLOCK) void k_radix_scatter(const uint32_t* __restrict__ keys,
                                                               const uint32_t* __restrict__ vals, uint32_t n,
                                                               const uint32_t* __restrict__ count, uint32_t shift,
-                                                              const uint32_t* __restrict__ offsets, uint32_t tiles,
+                                                              const uint32_t* __restrict__ offsets,
+                                                              const uint32_t* __restrict__ totals, uint32_t tiles,
                                                               uint32_t* __restrict__ keys_out,
                                                               uint32_t* __restrict__ vals_out) {
     __shared__ uint32_t s_key[SORT_TILE];
@@ -374,7 +348,9 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_radix_scatter(const uint32_t* __
     }
     uint32_t total;
     const uint32_t first = block_inclusive_scan(total_of_digit, wsum, &total) - total_of_digit;
-    out_base[threadIdx.x] = offsets[threadIdx.x * tiles + blockIdx.x] - first;
+    const uint32_t items = totals[threadIdx.x];  // of all tiles
+    const uint32_t start = block_inclusive_scan(items, wsum, &total) - items;
+    out_base[threadIdx.x] = start + offsets[threadIdx.x * tiles + blockIdx.x] - first;
 #pragma unroll
     for (int w = 0; w < SORT_WAVES; ++w) wave_cnt[w][threadIdx.x] += first;
     __syncthreads();
@@ -392,6 +368,110 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_radix_scatter(const uint32_t* __
         const uint32_t dst = out_base[(k >> shift) & (RADIX - 1)] + i;
         if (keys_out) keys_out[dst] = k;
         vals_out[dst] = s_val[i];
+    }
+}
+
+// The whole sort of at most SMALL_KEYS pairs by one workgroup, in place: the
+// pairs stay in LDS, and every pass ranks them as the scatter ranks a tile. A
+// pass is then a few barriers instead of three launches: 4,404 keys take 21 us,
+// as four passes over the device 78 (their launches fill it with three blocks).
+constexpr int SMALL_BLOCK = 1024;
+constexpr int SMALL_WAVES = SMALL_BLOCK / 64;
+constexpr int SMALL_ITEMS = 8;
+constexpr uint32_t SMALL_KEYS = SMALL_BLOCK * SMALL_ITEMS;
+
+__global__ __launch_bounds__(SMALL_BLOCK) void k_small_sort(uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                            uint32_t n, uint32_t bits) {
+    __shared__ uint32_t s_key[SMALL_KEYS], s_val[SMALL_KEYS];
+    __shared__ uint32_t wave_cnt[SMALL_WAVES][RADIX];
+    __shared__ uint32_t wsum[RADIX / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    uint32_t key[SMALL_ITEMS], val[SMALL_ITEMS], pos[SMALL_ITEMS];
+    const uint32_t items = (n + SMALL_BLOCK - 1) / SMALL_BLOCK;  // rounds in use: fewer keys, shorter waves' stretches
+    const uint32_t base = wave * items * 64 + lane;
+#pragma unroll
+    for (int r = 0; r < SMALL_ITEMS; ++r) {
+        const uint32_t idx = base + 64 * r;
+        const bool valid = r < (int)items && idx < n;
+        key[r] = valid ? keys[idx] : 0u;
+        val[r] = valid ? vals[idx] : 0u;
+    }
+    uint32_t* cnt = wave_cnt[wave];
+    for (uint32_t shift = 0; shift < bits; shift += 8) {
+#pragma unroll
+        for (int k = 0; k < RADIX / 64; ++k) cnt[64 * k + lane] = 0;
+#pragma unroll
+        for (int r = 0; r < SMALL_ITEMS; ++r) {
+            if (r >= (int)items) break;
+            const bool valid = base + 64 * r < n;
+            const uint32_t digit = (key[r] >> shift) & (RADIX - 1);
+            uint64_t same = __ballot(valid);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (digit >> b) & 1u;
+                const uint64_t m = __ballot(bit);
+                same &= bit ? m : ~m;
+            }
+            const uint32_t rank = __popcll(same & lt_mask);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const uint32_t before = cnt[digit];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (valid && rank == 0) cnt[digit] = before + (uint32_t)__popcll(same);
+            pos[r] = before + rank;
+        }
+        __syncthreads();
+        // per digit (one of the first 256 threads): the waves one after another
+        uint32_t all = 0, incl = 0;
+        if (threadIdx.x < RADIX) {
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; ++w) {
+                const uint32_t t = wave_cnt[w][threadIdx.x];
+                wave_cnt[w][threadIdx.x] = all;
+                all += t;
+            }
+            incl = all;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t t = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += t;
+            }
+            if (lane == 63) wsum[wave] = incl;
+        }
+        __syncthreads();
+        if (threadIdx.x < RADIX) {
+            uint32_t first = incl - all;
+            for (int w = 0; w < wave; ++w) first += wsum[w];
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; ++w) wave_cnt[w][threadIdx.x] += first;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < SMALL_ITEMS; ++r) {
+            if (r < (int)items && base + 64 * r < n) {
+                const uint32_t at = cnt[(key[r] >> shift) & (RADIX - 1)] + pos[r];
+                s_key[at] = key[r];
+                s_val[at] = val[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < SMALL_ITEMS; ++r) {
+            const uint32_t idx = base + 64 * r;
+            if (r < (int)items && idx < n) {
+                key[r] = s_key[idx];
+                val[r] = s_val[idx];
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < SMALL_ITEMS; ++r) {
+        const uint32_t idx = base + 64 * r;
+        if (r < (int)items && idx < n) {
+            keys[idx] = key[r];
+            vals[idx] = val[r];
+        }
     }
 }
 
@@ -945,43 +1025,32 @@ inline uint32_t blocks_for(size_t n, int block) { return (uint32_t)((n + block -
 
 }  // namespace
 
-// Exclusive prefix sum of `count` device words in place; `partials` holds
-// ceil(count / 2048) words of scratch.
-lucida_status scan_u32_device(lucida_ctx* ctx, uint32_t* data, uint32_t count, uint32_t* partials) {
-    if (count == 0) return LUCIDA_OK;
-    const uint32_t segs = blocks_for(count, SCAN_SEG);
-    hipLaunchKernelGGL(k_scan_reduce, dim3(segs), dim3(SCAN_BLOCK), 0, ctx->stream, data, count, partials);
-    hipLaunchKernelGGL(k_scan_down, dim3(segs), dim3(SCAN_BLOCK), 0, ctx->stream, data, count, partials);
-    LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
-    return LUCIDA_OK;
-}
-
-// Words of histogram + scan scratch a sort of n keys uses.
-static size_t sort_scratch_words(size_t n) {
-    const size_t hist_words = blocks_for(n, SORT_TILE) * (size_t)RADIX;
-    return hist_words + blocks_for(hist_words, SCAN_SEG);
-}
+// Words of histogram and digit totals a sort of n keys uses.
+static size_t sort_scratch_words(size_t n) { return (blocks_for(n, SORT_TILE) + (size_t)1) * RADIX; }
 
 // Radix-sorts device arrays keys/vals in place over bits [0, bits), using
 // tmp arrays of the same length and `work` (sort_scratch_words(n) words,
 // every word written before it is read, so it needs no clearing).
 static lucida_status sort_device_with(lucida_ctx* ctx, uint32_t* keys, uint32_t* vals, uint32_t* tk, uint32_t* tv,
                                       size_t n, uint32_t bits, uint32_t* work) {
+    if (n <= SMALL_KEYS) {
+        hipLaunchKernelGGL(k_small_sort, dim3(1), dim3(SMALL_BLOCK), 0, ctx->stream, keys, vals, (uint32_t)n,
+                           (bits + 7) / 8 * 8);
+        LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
+        return LUCIDA_OK;
+    }
     const uint32_t tiles = blocks_for(n, SORT_TILE);
-    const uint32_t hist_words = tiles * RADIX;
-    const uint32_t segs = blocks_for(hist_words, SCAN_SEG);
     uint32_t* hist = work;
-    uint32_t* partials = hist + hist_words;
+    uint32_t* totals = hist + (size_t)tiles * RADIX;
     uint32_t *src_k = keys, *src_v = vals, *dst_k = tk, *dst_v = tv;
     const uint32_t passes = (bits + 7) / 8;
     for (uint32_t pass = 0; pass < passes; ++pass) {
         const uint32_t shift = pass * 8;
         hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(SORT_BLOCK), 0, ctx->stream, src_k, (uint32_t)n,
                            nullptr, shift, hist, tiles);
-        hipLaunchKernelGGL(k_scan_reduce, dim3(segs), dim3(SCAN_BLOCK), 0, ctx->stream, hist, hist_words, partials);
-            hipLaunchKernelGGL(k_scan_down, dim3(segs), dim3(SCAN_BLOCK), 0, ctx->stream, hist, hist_words, partials);
+        hipLaunchKernelGGL(k_scan_rows, dim3(RADIX), dim3(SCAN_BLOCK), 0, ctx->stream, hist, tiles, totals);
         hipLaunchKernelGGL(k_radix_scatter, dim3(tiles), dim3(SORT_BLOCK), 0, ctx->stream, src_k, src_v,
-                           (uint32_t)n, nullptr, shift, hist, tiles, dst_k, dst_v);
+                           (uint32_t)n, nullptr, shift, hist, totals, tiles, dst_k, dst_v);
         std::swap(src_k, dst_k);
         std::swap(src_v, dst_v);
     }
@@ -1005,17 +1074,15 @@ static lucida_status sort_device(lucida_ctx* ctx, uint32_t* keys, uint32_t* vals
 // ---------------------------------------------------------------------------
 // Sort scratch that is never allocated: a file-scope device array, one copy
 // per GPU, for callers that cannot allocate (code under graph capture, tight
-// serving loops). 8 MiB + 4 KiB covers LUCIDA_SORT_NOALLOC_MAX_KEYS keys.
+// serving loops). 8 MiB + 1 KiB covers LUCIDA_SORT_NOALLOC_MAX_KEYS keys.
 // Host code never passes `scratch` itself (its host-side name is not a
 // device address): each device's address comes from hipGetSymbolAddress,
 // made once per device with that device current, and is kept in
 // g_scratch_ptr.
 // ---------------------------------------------------------------------------
 
-constexpr size_t SORT_NOALLOC_WORDS =
-    (LUCIDA_SORT_NOALLOC_MAX_KEYS / SORT_TILE) * RADIX + (LUCIDA_SORT_NOALLOC_MAX_KEYS / SORT_TILE) * RADIX / SCAN_SEG;
+constexpr size_t SORT_NOALLOC_WORDS = (LUCIDA_SORT_NOALLOC_MAX_KEYS / SORT_TILE + 1) * RADIX;
 static_assert(LUCIDA_SORT_NOALLOC_MAX_KEYS % SORT_TILE == 0, "max keys is a whole number of tiles");
-static_assert((LUCIDA_SORT_NOALLOC_MAX_KEYS / SORT_TILE) * RADIX % SCAN_SEG == 0, "whole scan segments");
 
 static __device__ __align__(256) uint32_t scratch[SORT_NOALLOC_WORDS];
 
@@ -1038,10 +1105,7 @@ lucida_status sort_scratch_init(lucida_ctx* ctx) {
     return LUCIDA_OK;
 }
 
-size_t sort_counted_scratch_words(size_t capacity) {
-    const size_t hist_words = blocks_for(capacity, SORT_TILE) * (size_t)RADIX;
-    return hist_words + blocks_for(hist_words, SCAN_SEG);
-}
+size_t sort_counted_scratch_words(size_t capacity) { return sort_scratch_words(capacity); }
 
 // Stable sort of (keys, vals)[0, *count) by key bits [0, bits) on `stream`,
 // bits a multiple of 8 (one pass per 8 bits). The count stays on the device:
@@ -1059,19 +1123,17 @@ lucida_status sort_pairs_counted(hipStream_t stream, uint32_t* keys, uint32_t* v
     if (bits == 0 || bits % 8 != 0 || bits > 32) return set_error(LUCIDA_INVALID_ARG, "sort: bits must be 8, 16, 24 or 32");
     if (capacity > 0xFFFFFFFFull / 2) return set_error(LUCIDA_INVALID_ARG, "sort: more than 2^31 keys");
     const uint32_t tiles = blocks_for(capacity, SORT_TILE);
-    const uint32_t hist_words = tiles * RADIX;
-    const uint32_t segs = blocks_for(hist_words, SCAN_SEG);
     uint32_t* hist = work;
-    uint32_t* partials = work + hist_words;
+    uint32_t* totals = hist + (size_t)tiles * RADIX;
     uint32_t *src_k = keys, *src_v = vals, *dst_k = tk, *dst_v = tv;
     for (uint32_t shift = 0; shift < bits; shift += 8) {
         hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(SORT_BLOCK), 0, stream, src_k, (uint32_t)capacity, count,
                            shift, hist, tiles);
-        hipLaunchKernelGGL(k_scan_reduce, dim3(segs), dim3(SCAN_BLOCK), 0, stream, hist, hist_words, partials);
-        hipLaunchKernelGGL(k_scan_down, dim3(segs), dim3(SCAN_BLOCK), 0, stream, hist, hist_words, partials);
+        hipLaunchKernelGGL(k_scan_rows, dim3(RADIX), dim3(SCAN_BLOCK), 0, stream, hist, tiles, totals);
         // the last pass needs only the values
         hipLaunchKernelGGL(k_radix_scatter, dim3(tiles), dim3(SORT_BLOCK), 0, stream, src_k, src_v,
-                           (uint32_t)capacity, count, shift, hist, tiles, shift + 8 < bits ? dst_k : nullptr, dst_v);
+                           (uint32_t)capacity, count, shift, hist, totals, tiles, shift + 8 < bits ? dst_k : nullptr,
+                           dst_v);
         std::swap(src_k, dst_k);
         std::swap(src_v, dst_v);
     }
