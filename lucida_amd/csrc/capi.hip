@@ -133,6 +133,7 @@ void lucida_ctx_destroy(lucida_ctx* ctx) {
                       &ctx->conv_buf, &ctx->mk_spill, &ctx->mk_state,  &ctx->tl_cost,   &ctx->tl_leafy,
                       &ctx->tl_order,  &ctx->tl_list};
     for (DevBuf* b : bufs) b->release();
+    if (ctx->lb_host) (void)hipHostFree(ctx->lb_host);
     if (ctx->tl_host) (void)hipHostFree(ctx->tl_host);
     if (ctx->tl_counted) (void)hipEventDestroy(ctx->tl_counted);
     for (WfPipe& w : ctx->wf) {

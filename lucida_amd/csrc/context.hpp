@@ -99,6 +99,7 @@ struct lucida_ctx {
     // LBVH scratch, reused between builds.
     lucida::DevBuf lb_bounds, lb_partial, lb_codes, lb_vals, lb_tmpk, lb_tmpv, lb_hist, lb_karras, lb_parent,
         lb_nodebox, lb_subtree, lb_flags, lb_misc, lb_rank, lb_nodes, lb_tris, lb_pos, lb_prims, lb_level;
+    uint32_t* lb_host = nullptr;  // a build's node count word, in pinned host memory
     // Treelet restructuring: per-node costs, leaf choices, the leaf order.
     lucida::DevBuf tl_cost, tl_leafy, tl_order, tl_list;
     uint32_t* tl_host = nullptr;       // a round's per-level counts, in pinned host memory,
