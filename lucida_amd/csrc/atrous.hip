@@ -85,7 +85,8 @@ constexpr float LOG2E = 1.4426950408889634f;
 // wide strides need no taller tile. Pixels outside the image get a zero
 // normal, hence weight zero. FIRST (S = 1) reads the film itself, makes the
 // guides and the 3x3 luminance deviation (denoise.rs:111) and stores them for
-// the later passes; LAST writes the remodulated result.
+// the later passes; LAST writes the remodulated result (a job without an output
+// film leaves the demodulated one in the plane).
 //
 // The edge stops multiply to one exponential with the kernel's weight: K *
 // nd^s * e^-(a+b+c) = 2^(log2 K + s*log2(nd) - (a+b+c)*log2(e)), with the
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(DN_THREADS) void k_dn_tile(DnJobs jobs, DnPlanes pl
         r.z = sz / ws;
         r.w = lum3(r.x, r.y, r.z);
     }
-    if (LAST)
+    if (LAST && J.out)
         dn_write(J.out + i, r, dn_albedo(J.in + i), cg);
     else
         pl.b[J.base + i] = r;
@@ -296,7 +297,7 @@ __global__ __launch_bounds__(TX* TY) void k_dn_pass(DnJobs jobs, DnPlanes pl, in
         r.z = sz / ws;
         r.w = lum3(r.x, r.y, r.z);
     }
-    if (last)
+    if (last && J.out)
         dn_write(J.out + ci, r, dn_albedo(J.in + ci), cg);
     else
         pl.b[J.base + ci] = r;
@@ -338,7 +339,9 @@ lucida_status atrous_reserve(lucida_ctx* ctx, size_t pixels) {
 
 // Queues the filter of `count` Accum films on the context's stream, film k into
 // `out[k]`; the planes must have been reserved for the films' pixels together.
-void atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuAccum* const* out, size_t count,
+// With a null `out` (and at least one iteration) the demodulated colours stay in
+// a plane of the context, film after film, until its next filter; returned.
+const float4* atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuAccum* const* out, size_t count,
                     const lucida_denoise_params& params) {
     size_t n = 0;
     for (size_t k = 0; k < count; ++k) n += (size_t)in[k]->width * in[k]->height;
@@ -350,13 +353,14 @@ void atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuAccum* con
     pl.dev = pl.alum + n;
     hipStream_t s = ctx->stream;
     size_t base = 0;
+    const float4* result = params.iterations % 2 ? pl.b : pl.a;  // the last pass's plane
     for (size_t first = 0; first < count; first += DN_JOBS) {
         const unsigned jn = (unsigned)std::min<size_t>(DN_JOBS, count - first);
         DnJobs jobs{};
         uint32_t w = 0, h = 0;
         for (unsigned k = 0; k < jn; ++k) {
             const lucida_film* f = in[first + k];
-            jobs.job[k] = DnJob{f->accum, out[first + k], f->width, f->height, (uint32_t)base, 0u};
+            jobs.job[k] = DnJob{f->accum, out ? out[first + k] : nullptr, f->width, f->height, (uint32_t)base, 0u};
             base += (size_t)f->width * f->height;
             w = std::max(w, f->width);
             h = std::max(h, f->height);
@@ -383,6 +387,7 @@ void atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuAccum* con
             std::swap(p.a, p.b);
         }
     }
+    return result;
 }
 
 }  // namespace lucida

@@ -181,8 +181,9 @@ lucida_status build_prim_planes(lucida_ctx* ctx, lucida_scene* scene);
 lucida_status build_tri_edges(lucida_ctx* ctx, lucida_scene* scene);
 // A-trous filter (atrous.hip) without the final wait: reserve the planes for
 // the films' pixels together first, then queue their filters on the context's
-// stream, film k into out[k].
+// stream, film k into out[k], or (out null) the demodulated colours into a
+// plane, film after film, which is returned and holds until the next filter.
 lucida_status atrous_reserve(lucida_ctx* ctx, size_t pixels);
-void atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuAccum* const* out, size_t count,
+const float4* atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuAccum* const* out, size_t count,
                     const lucida_denoise_params& params);
 }  // namespace lucida

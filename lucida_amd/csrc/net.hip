@@ -634,10 +634,13 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(const float* __restrict__ par
 // albedo so inference can remodulate with the same guide.
 //
 // One launch serves up to FEATURE_FILMS films (blockIdx.z): each one's filtered
-// and reference films, row width and crop origin, and its place in the batch.
+// colours and reference film, row width and crop origin, and its place in the
+// batch. The filtered colours are read from the filter's own plane, 16 bytes a
+// pixel: as an Accum film they were 64 written and a line of 64 read.
 constexpr int FEATURE_FILMS = 16;
 struct FeatureFilm {
-    const GpuAccum *film, *base, *ref;
+    const GpuAccum *film, *ref;
+    const float4* base;  // the demodulated a-trous estimate, per pixel of the film
     int fw, x0, y0, img;
 };
 struct FeatureFilms {
@@ -649,7 +652,7 @@ __global__ void k_features(FeatureFilms films, int cw, int ch, bf16* __restrict_
     const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
     if (x >= cw || y >= ch) return;
     const FeatureFilm& F = films.film[blockIdx.z];
-    const GpuAccum *film = F.film, *base = F.base, *ref = F.ref;
+    const GpuAccum *film = F.film, *ref = F.ref;
     const int fw = F.fw, x0 = F.x0, y0 = F.y0, img = F.img;
     const size_t src = (size_t)(y0 + y) * fw + (x0 + x);
     const float4* a = reinterpret_cast<const float4*>(film + src);
@@ -676,11 +679,10 @@ __global__ void k_features(FeatureFilms films, int cw, int ch, bf16* __restrict_
     f[11] = log2f(ns) * (1.0f / 16.0f);
     // The a-trous estimate of the same film, demodulated like channels 0..2:
     // the network predicts a correction to it.
-    const float4 b0 = reinterpret_cast<const float4*>(base + src)[0];
-    const float binv = 1.0f / fmaxf(b0.w, 1.0f);
-    f[12] = log1pf(fmaxf(b0.x * binv / al[0], 0.0f));
-    f[13] = log1pf(fmaxf(b0.y * binv / al[1], 0.0f));
-    f[14] = log1pf(fmaxf(b0.z * binv / al[2], 0.0f));
+    const float4 b0 = F.base[src];  // remodulated as the filter's film is, then demodulated
+    f[12] = log1pf(fmaxf(b0.x * al[0] / al[0], 0.0f));
+    f[13] = log1pf(fmaxf(b0.y * al[1] / al[1], 0.0f));
+    f[14] = log1pf(fmaxf(b0.z * al[2] / al[2], 0.0f));
     f[15] = 0.0f;
     const size_t dst = ((size_t)img * ch + y) * cw + x;
     // The estimate the output corrects, kept in FP32: in BF16 (8 significant
@@ -773,7 +775,7 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ grad, fl
 const lucida_denoise_params kAtrousDefaults = {4u, 64.0f, 0.08f, 4.0f, 0.1f};
 
 // Films filtered together for a batch's features, by their pixels: enough to
-// fill the device, while the filter's planes and results stay near 500 MB.
+// fill the device, while the filter's planes stay near 240 MB.
 constexpr size_t NET_FILTER_PIXELS = (size_t)1 << 22;
 
 inline unsigned grid1(size_t n, int block = 256) {
@@ -918,8 +920,7 @@ struct lucida_net {
     DevBuf frag_fwd, frag_bwd;             // bf16 fragments
     size_t frag_fwd_off[kNetNumLayers], frag_bwd_off[kNetNumLayers], param_off[kNetNumLayers];
     DevBuf acts, dacts, target, loss_partial;
-    DevBuf base;  // a-trous estimates of the films being loaded (Accum-shaped)
-    DevBuf base_log;  // its log1p(estimate / albedo) per pixel of the batch, FP32 (3 floats)
+    DevBuf base_log;  // log1p(a-trous estimate / albedo) per pixel of the batch, FP32 (3 floats)
     size_t act_capacity = 0;
     // a gradient ready for its weight gradient; the weight gradients done
     hipEvent_t ev_ready = nullptr, ev_done = nullptr;
@@ -1187,7 +1188,7 @@ void lucida_net_destroy(lucida_net* net) {
     if (net->ev_ready) (void)hipEventDestroy(net->ev_ready);
     if (net->ev_done) (void)hipEventDestroy(net->ev_done);
     DevBuf* b[] = {&net->params, &net->grads, &net->adam_m, &net->adam_v, &net->frag_fwd, &net->frag_bwd,
-                   &net->acts, &net->dacts, &net->target, &net->loss_partial, &net->base, &net->base_log,
+                   &net->acts, &net->dacts, &net->target, &net->loss_partial, &net->base_log,
                    &net->wg_part};
     for (DevBuf* x : b) x->release();
     delete net;
@@ -1229,7 +1230,7 @@ static lucida_status load_batch(lucida_net* net, const lucida_film* const* input
     lucida_status st = net_ensure_acts(net, (int)count, (int)h, (int)w);
     if (st != LUCIDA_OK) return st;
     // Whole films are filtered (crops then see the filter's real neighbourhood),
-    // as many together as make NET_FILTER_PIXELS, each into its part of `base`.
+    // as many together as make NET_FILTER_PIXELS.
     auto pixels_of = [&](uint32_t k) { return (size_t)inputs[k]->width * inputs[k]->height; };
     auto group_end = [&](uint32_t first, size_t* pixels) {
         uint32_t k = first;
@@ -1242,31 +1243,22 @@ static lucida_status load_batch(lucida_net* net, const lucida_film* const* input
         k = group_end(k, &group);
         max_pixels = std::max(max_pixels, group);
     }
-    if (max_pixels * sizeof(GpuAccum) > net->base.bytes) {
-        LUCIDA_HIP(hipStreamSynchronize(net->ctx->stream), LUCIDA_VALIDATION);
-        LUCIDA_HIP(net->base.ensure(max_pixels * sizeof(GpuAccum)), LUCIDA_OOM);
-    }
     st = atrous_reserve(net->ctx, max_pixels);
     if (st != LUCIDA_OK) return st;
     const ActPlan a = plan_acts(net->n, net->h, net->w);
     bf16* X = net->acts.as<bf16>() + a.x;
-    std::vector<GpuAccum*> filtered;
     for (uint32_t first = 0; first < count;) {
         const uint32_t end = group_end(first, &group);
-        filtered.clear();
-        GpuAccum* at = net->base.as<GpuAccum>();
-        for (uint32_t k = first; k < end; ++k) {
-            filtered.push_back(at);
-            at += pixels_of(k);
-        }
-        atrous_enqueue(net->ctx, inputs + first, filtered.data(), end - first, kAtrousDefaults);
+        const float4* filtered = atrous_enqueue(net->ctx, inputs + first, nullptr, end - first, kAtrousDefaults);
         for (uint32_t f0 = first; f0 < end; f0 += FEATURE_FILMS) {
             FeatureFilms ff{};
             const uint32_t n = std::min<uint32_t>(FEATURE_FILMS, end - f0);
-            for (uint32_t k = 0; k < n; ++k)
-                ff.film[k] = FeatureFilm{inputs[f0 + k]->accum, filtered[f0 + k - first],
-                                         refs ? refs[f0 + k]->accum : nullptr, (int)inputs[f0 + k]->width,
-                                         x0 ? (int)x0[f0 + k] : 0, y0 ? (int)y0[f0 + k] : 0, (int)(f0 + k)};
+            for (uint32_t k = 0; k < n; ++k) {
+                ff.film[k] = FeatureFilm{inputs[f0 + k]->accum, refs ? refs[f0 + k]->accum : nullptr, filtered,
+                                         (int)inputs[f0 + k]->width, x0 ? (int)x0[f0 + k] : 0,
+                                         y0 ? (int)y0[f0 + k] : 0, (int)(f0 + k)};
+                filtered += pixels_of(f0 + k);
+            }
             hipLaunchKernelGGL(k_features, dim3((w + 127) / 128, h, n), dim3(128), 0, net->ctx->stream, ff, (int)w,
                                (int)h, X, net->base_log.as<float>(), refs ? net->target.as<float>() : nullptr);
         }
