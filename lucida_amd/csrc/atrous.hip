@@ -102,6 +102,7 @@ constexpr float LOG2E = 1.4426950408889634f;
 // and 61 at 256 x 256; eight rows a block 136 and 37.
 constexpr int DN_W = 64, DN_ROWS = 4;
 constexpr int DN_THREADS = DN_W * DN_ROWS;
+constexpr uint32_t DN_MAX_H = 200000;  // tiles of taller films would not fit a grid's y
 
 template <int S, bool FIRST, bool LAST>
 __global__ __launch_bounds__(DN_THREADS) void k_dn_tile(DnJobs jobs, DnPlanes pl, lucida_denoise_params prm) {
@@ -214,8 +215,8 @@ __global__ __launch_bounds__(DN_THREADS) void k_dn_tile(DnJobs jobs, DnPlanes pl
 }
 
 // The passes that tiles do not serve (strides of 16 and more, whose halo is
-// the larger part of a tile, and normal stops that are not positive) read
-// each tap from the planes.
+// the larger part of a tile, normal stops that are not positive, and films of
+// more rows than a grid takes) read each tap from the planes.
 
 // The first pass's planes from the film.
 __global__ __launch_bounds__(TX* TY) void k_dn_prepare(DnJobs jobs, DnPlanes pl) {
@@ -370,7 +371,7 @@ const float4* atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuA
             hipLaunchKernelGGL(k_dn_modulate, grd, blk, 0, s, jobs);
             continue;
         }
-        const bool tiles = params.sigma_normal > 0.0f;
+        const bool tiles = params.sigma_normal > 0.0f && h <= DN_MAX_H;
         DnPlanes p = pl;
         if (!tiles) {
             hipLaunchKernelGGL(k_dn_prepare, grd, blk, 0, s, jobs, p);
