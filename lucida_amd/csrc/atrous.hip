@@ -102,7 +102,9 @@ constexpr float LOG2E = 1.4426950408889634f;
 // and 61 at 256 x 256; eight rows a block 136 and 37.
 constexpr int DN_W = 64, DN_ROWS = 4;
 constexpr int DN_THREADS = DN_W * DN_ROWS;
-constexpr uint32_t DN_MAX_H = 200000;  // tiles of taller films would not fit a grid's y
+// A grid's y holds 65,535 blocks; 200,000 rows take about 50,000 of 4 rows at
+// any stride, and taller films keep the untiled passes (25,000 blocks of 8).
+constexpr uint32_t DN_MAX_H = 200000;
 
 template <int S, bool FIRST, bool LAST>
 __global__ __launch_bounds__(DN_THREADS) void k_dn_tile(DnJobs jobs, DnPlanes pl, lucida_denoise_params prm) {

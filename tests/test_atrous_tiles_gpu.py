@@ -1,7 +1,7 @@
 """The a-trous filter's tiles at the sizes where they can go wrong: films
 narrower than a tile or than a stride's halo, odd sides, every stride with
-tiles and without, a first pass that is also the last, and the options that
-keep to the untiled passes."""
+tiles and without, a first pass that is also the last, and the options and
+heights that keep to the untiled passes."""
 from __future__ import annotations
 
 import numpy as np
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 # (width, height, iterations, sigma_normal)
 CASES = [(1, 1, 4, 64.0), (3, 130, 4, 64.0), (130, 3, 4, 64.0), (64, 16, 1, 64.0), (65, 17, 2, 64.0), (127, 67, 3, 64.0),
-         (200, 129, 4, 64.0), (97, 133, 6, 64.0), (70, 40, 4, 0.0), (70, 40, 5, 8.0)]
+         (200, 129, 4, 64.0), (97, 133, 6, 64.0), (70, 40, 4, 0.0), (70, 40, 5, 8.0),
+         (3, 200000, 4, 64.0), (3, 200001, 4, 64.0)]
 
 
 @pytest.mark.parametrize("w,h,iterations,sigma_normal", CASES)
