@@ -88,18 +88,26 @@ constexpr float LOG2E = 1.4426950408889634f;
 // the later passes; LAST writes the remodulated result (a job without an output
 // film leaves the demodulated one in the plane).
 //
-// The edge stops multiply to one exponential with the kernel's weight: K *
-// nd^s * e^-(a+b+c) = 2^(log2 K + s*log2(nd) - (a+b+c)*log2(e)), with the
-// stops' reciprocals taken once per pixel and the hardware's exp2 / log2 (a
-// relative error near 1e-6 in a weight); s > 0.
+// The edge stops multiply to one exponential: nd^s * e^-(a+b+c) =
+// 2^(s*log2(nd) - (a+b+c)*log2(e)), with the stops' reciprocals taken once per
+// pixel and the hardware's exp2 / log2 (a relative error near 1e-6 in a
+// weight); every stop must be positive. The hardware's exp2 gives no
+// subnormals, so the kernel's factor stays outside it: as part of the exponent
+// it made weights vanish that are up to 2^8 times the least. The terms and the
+// sums are those of k_dn_pass in its order, so a film's result does not depend
+// on which of the two filters it (a pixel outside adds zeros).
 //
-// What bounds it: about 24 vector instructions and 36 bytes of LDS a tap, two of
-// the instructions at a quarter of the rate, and the latency of the staging
-// loads. Four passes and their preparation at 1024 x 1024: 133 us, at 256 x
-// 256: 36; with every tap read through L1 and the preparation apart, 346 and
-// 43. Two or four rows a thread (each tap read from LDS once for all of them)
-// save LDS reads but leave too few waves for the latency: 140 and 145 us, 43
-// and 61 at 256 x 256; eight rows a block 136 and 37.
+// What bounds it: vector issue. A tap takes 35 vector instructions, two of them
+// at a quarter of the rate; a middle pass at 1024 x 1024 takes 28 us, of which
+// the SIMDs issue them for 25, and its LDS reads wait for few bank conflicts
+// (0.1M cycles over all CUs). Whole calls at 1024 x 1024: 132 to 142 us, at
+// 256 x 256: 37; with every tap read through L1 and the preparation apart, 344 to
+// 354 and 54. Fused multiply-adds and the kernel's factor in the exponent would
+// take 124 and 35, but give other sums than the untiled passes and lose small
+// weights. In that form two or four rows a thread (each tap read from LDS once
+// for all of them) left too few waves for the latency: 140 and 145 us against
+// 133 on one run, 43 and 61 against 36 at 256 x 256; eight rows a block 136 and
+// 37.
 constexpr int DN_W = 64, DN_ROWS = 4;
 constexpr int DN_THREADS = DN_W * DN_ROWS;
 // A grid's y holds 65,535 blocks; 200,000 rows take about 50,000 of 4 rows at
@@ -178,28 +186,24 @@ __global__ __launch_bounds__(DN_THREADS) void k_dn_tile(DnJobs jobs, DnPlanes pl
     const float rl = LOG2E / (prm.sigma_luminance * fmaxf(d, 1.0e-4f));
     const float ra = LOG2E / (prm.sigma_albedo * ca);
     const float sn = prm.sigma_normal;
-    // log2 of the kernel 1/16, 1/4, 3/8, 1/4, 1/16 (denoise.rs)
-    constexpr float LK0 = -4.0f, LK1 = -2.0f, LK2 = -1.4150374992788437f;
     float sx = 0.0f, sy = 0.0f, sz = 0.0f, ws = 0.0f;
 #pragma unroll 1
-    for (int kx = 0; kx < 5; ++kx) {
-        const float lkx = kx == 2 ? LK2 : (kx == 1 || kx == 3 ? LK1 : LK0);
-        const int col = ty * PITCH + tx + kx * S;
+    for (int ky = 0; ky < 5; ++ky) {
+        const float kr = ky == 2 ? 3.0f / 8.0f : (ky == 1 || ky == 3 ? 1.0f / 4.0f : 1.0f / 16.0f);
+        const float k0 = 1.0f / 16.0f * kr, k1 = 1.0f / 4.0f * kr, k2 = 3.0f / 8.0f * kr;
+        const int row = (ty + ky) * PITCH + tx;
 #pragma unroll
-        for (int ky = 0; ky < 5; ++ky) {
-            const float4 qg = s_gnd[col + ky * PITCH];
-            const float4 qc = s_col[col + ky * PITCH];
-            const float qa = s_alb[col + ky * PITCH];
-            const float lk = lkx + (ky == 2 ? LK2 : (ky == 1 || ky == 3 ? LK1 : LK0));
-            const float nd = fmaxf(fmaf(cg.z, qg.z, fmaf(cg.y, qg.y, cg.x * qg.x)), 0.0f);
-            float e = fmaf(sn, __builtin_amdgcn_logf(nd), lk);  // -inf at nd = 0
-            e = fmaf(-fabsf(cg.w - qg.w), rd, e);
-            e = fmaf(-fabsf(cl - qc.w), rl, e);
-            e = fmaf(-fabsf(ca - qa), ra, e);
-            const float wt = __builtin_amdgcn_exp2f(e);
-            sx = fmaf(qc.x, wt, sx);
-            sy = fmaf(qc.y, wt, sy);
-            sz = fmaf(qc.z, wt, sz);
+        for (int kx = 0; kx < 5; ++kx) {
+            const float4 qg = s_gnd[row + kx * S];
+            const float4 qc = s_col[row + kx * S];
+            const float qa = s_alb[row + kx * S];
+            const float nd = fmaxf(cg.x * qg.x + cg.y * qg.y + cg.z * qg.z, 0.0f);
+            const float ln = sn * __builtin_amdgcn_logf(nd);  // -inf at nd = 0
+            const float e = ln - fabsf(cg.w - qg.w) * rd - fabsf(cl - qc.w) * rl - fabsf(ca - qa) * ra;
+            const float wt = (kx == 2 ? k2 : (kx == 1 || kx == 3 ? k1 : k0)) * __builtin_amdgcn_exp2f(e);
+            sx += qc.x * wt;
+            sy += qc.y * wt;
+            sz += qc.z * wt;
             ws += wt;
         }
     }
@@ -217,8 +221,8 @@ __global__ __launch_bounds__(DN_THREADS) void k_dn_tile(DnJobs jobs, DnPlanes pl
 }
 
 // The passes that tiles do not serve (strides of 16 and more, whose halo is
-// the larger part of a tile, normal stops that are not positive, and films of
-// more rows than a grid takes) read each tap from the planes.
+// the larger part of a tile, stops that are not positive, and films of more
+// rows than a grid takes) read each tap from the planes.
 
 // The first pass's planes from the film.
 __global__ __launch_bounds__(TX* TY) void k_dn_prepare(DnJobs jobs, DnPlanes pl) {
@@ -373,7 +377,9 @@ const float4* atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuA
             hipLaunchKernelGGL(k_dn_modulate, grd, blk, 0, s, jobs);
             continue;
         }
-        const bool tiles = params.sigma_normal > 0.0f && h <= DN_MAX_H;
+        // stops that are not positive could give a pixel outside the film a weight
+        const bool tiles = params.sigma_normal > 0.0f && params.sigma_depth > 0.0f && params.sigma_luminance > 0.0f &&
+                           params.sigma_albedo > 0.0f && h <= DN_MAX_H;
         DnPlanes p = pl;
         if (!tiles) {
             hipLaunchKernelGGL(k_dn_prepare, grd, blk, 0, s, jobs, p);
