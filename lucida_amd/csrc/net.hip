@@ -24,6 +24,7 @@
 
 #include "context.hpp"
 #include "net.hpp"
+#include "side_stream.hpp"
 
 namespace lucida {
 namespace {
@@ -1074,11 +1075,11 @@ static lucida_status net_backward(lucida_net* net) {
     // gradients, since neither fills the device at the coarse levels (training
     // step of eight 256 x 256 crops: 1.32 -> 1.25 ms).
     hipStream_t side = net->ctx->wf[0].s2;
+    SideStream beside(s, side, net->ev_ready, net->ev_done);
     for (int li = kNetNumLayers - 1; li >= 0; --li) {
         const NetLayer& L = kNetLayers[li];
         const int lvl = kNetLevel[li];
-        LUCIDA_HIP(hipEventRecord(net->ev_ready, s), LUCIDA_VALIDATION);
-        LUCIDA_HIP(hipStreamWaitEvent(side, net->ev_ready, 0), LUCIDA_VALIDATION);
+        LUCIDA_HIP(beside.fork(), LUCIDA_VALIDATION);
         const uint32_t row = (uint32_t)(9 * L.cin * L.cout + L.cout);  // the layer's W then b, as in `grads`
         lucida_status st = launch_wgrad(side, layer_source(A, a, li), D + a.l[li], L.cout, H0 >> lvl, W0 >> lvl, wg[li],
                                         net->wg_part.as<float>());
@@ -1107,8 +1108,7 @@ static lucida_status net_backward(lucida_net* net) {
         st = launch_conv(s, epi, c);
         if (st != LUCIDA_OK) return st;
     }
-    LUCIDA_HIP(hipEventRecord(net->ev_done, side), LUCIDA_VALIDATION);
-    LUCIDA_HIP(hipStreamWaitEvent(s, net->ev_done, 0), LUCIDA_VALIDATION);
+    LUCIDA_HIP(beside.join(), LUCIDA_VALIDATION);
     LUCIDA_HIP(hipGetLastError(), LUCIDA_SHADER);
     return LUCIDA_OK;
 }
