@@ -62,9 +62,11 @@ constexpr int lane_parts(int m) { return ((1 << (m - 1)) - 1 + (1 << LANE_SHIFT[
 constexpr int part_byte(int m) { return m == 2 ? 0 : part_byte(m - 1) + lane_parts(m - 1); }
 constexpr int SUBSET_BYTE = part_byte(LEAVES) + lane_parts(LEAVES);  // the lane's subsets of 2, 3, ... leaves
 static_assert(SUBSET_BYTE + LEAVES - 1 <= 32, "a lane's program is 32 bytes");
-struct LaneProgram {
+struct alignas(uint4) LaneProgram {  // a lane reads its 32 bytes as two uint4
     uint8_t byte[64][32];
 };
+static_assert(alignof(LaneProgram) >= alignof(uint4) && sizeof(LaneProgram::byte[0]) % sizeof(uint4) == 0,
+              "every lane's row is aligned for its loads");
 constexpr int popcount7(int v) { return (v & 1) + (v >> 1 & 1) + (v >> 2 & 1) + (v >> 3 & 1) + (v >> 4 & 1) + (v >> 5 & 1) + (v >> 6 & 1); }
 constexpr LaneProgram make_lane_program() {
     LaneProgram t{};
