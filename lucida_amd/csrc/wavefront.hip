@@ -47,12 +47,11 @@ constexpr int INST_STACK = 48;  // the two-level walk adds a RETURN marker and u
 constexpr int TRAV_BINARY = 0, TRAV_INSTANCED = 1;
 constexpr int MAX_BOUNCES = 64;
 // Counter words: queue length per bounce at [0, 72) (bounce b+1's count is
-// written by bounce b's SHADE), the rays PATHS traced at PATHS_AT, shadow-ray
-// count per bounce at [SHADOW_AT, +64), this batch's traversal counters (u64) at STATS_AT in STATS_STRIPES
+// written by bounce b's SHADE), shadow-ray count per bounce at [SHADOW_AT,
+// +64), this batch's traversal counters (u64) at STATS_AT in STATS_STRIPES
 // copies of 8 (a block adds to copy blockIdx % STATS_STRIPES, so the waves
 // of a launch do not queue on a few addresses), the render's running totals
 // (10 u64) at TOTALS_AT.
-constexpr uint32_t PATHS_AT = 72;  // extension and shadow rays traced by PATHS
 constexpr uint32_t SHADOW_AT = 80;
 constexpr uint32_t STATS_AT = 160;
 constexpr uint32_t STATS_STRIPES = 32;
@@ -832,12 +831,10 @@ __device__ inline bool analytic_any(const SceneView& sc, V3 o, V3 d, float t_max
 template <bool BATCH, int MODE>
 __global__ __launch_bounds__(TRACE_WG) void k_extend(SceneView sc0, const BatchJob* __restrict__ jobs, Planes p,
                                                      const uint32_t* __restrict__ queue,
-                                                     const uint32_t* __restrict__ count_ptr, uint32_t least,
-                                                     uint32_t stats_on) {
+                                                     const uint32_t* __restrict__ count_ptr, uint32_t stats_on) {
     __shared__ uint32_t stack_mem[LDS_STACK * TRACE_WG];
     const uint32_t i = blockIdx.x * TRACE_WG + threadIdx.x;
     const uint32_t count = *count_ptr;
-    if (count <= least) return;  // empty, or PATHS has it
     uint32_t visits = 0, tests = 0, overflow = 0;
     if (i < count) {
       RayStack st = make_stack(stack_mem, p.spill, MODE == TRAV_BINARY ? STACK : INST_STACK);
@@ -1151,10 +1148,9 @@ __global__ __launch_bounds__(SHADE_WG) void k_shade(SceneView sc0, const GpuUnif
                                               const uint32_t* __restrict__ queue_in,
                                               const uint32_t* __restrict__ count_ptr, uint32_t* __restrict__ queue_out,
                                               uint32_t* __restrict__ next_count, uint32_t* __restrict__ shadow_count,
-                                              uint32_t* __restrict__ key_out, Band band0, uint32_t least) {
+                                              uint32_t* __restrict__ key_out, Band band0) {
     const uint32_t i = blockIdx.x * SHADE_WG + threadIdx.x;
     const uint32_t count = *count_ptr;
-    if (count <= least) return;  // empty, or PATHS has it
     bool alive = false, shadow = false;
     uint32_t pid = 0, key = 0, skey = 0;
     ShadowRay sr{};
@@ -1453,62 +1449,24 @@ __global__ __launch_bounds__(TRACE_WG) void k_megakernel(SceneView sc, const Gpu
 //   instances-c3 (4,096)       5.52 / 4.32   6.04 / 5.01   6.01 / 5.29
 //   bvh-stress (368,640)       1.47 / 1.41   1.73 / 1.52   1.64 / 2.01
 // ---------------------------------------------------------------------------
-//
-// Without GEN it takes over a queue in the middle of a render, each path from
-// the bounce it stands at, if at most PATHS_TAIL are left: the same reasoning
-// for the last bounces, which last as long as ever with ever fewer rays. The
-// count is on the device only, so it is checked there: the launch returns if
-// the queue is longer, and EXTEND and SHADE of that bounce return if it is not,
-// as do the later bounces' (whose queues stay empty). A check costs its launch,
-// so there are two, where paths have thinned out but bounces remain, and only
-// two-level walks, whose chains are longest, repay the launches left empty:
-// instances-c3 640 x 360 x 4 spp 11.95 -> 9.71 ms, 960 x 540 x 4 14.57 -> 12.26,
-// 960 x 540 x 8 19.98 -> 19.32; but 640 x 360 x 1 (one band, nothing beside it)
-// 6.09 -> 6.41, 1024 x 1024 x 4 28.98 -> 29.15, cornell-mesh 640 x 360 x 4
-// 2.40 -> 2.42 and x 1 1.14 -> 1.30. So: instanced scenes, 2^18 to 2^21 paths
-// a band or batch.
 constexpr size_t PATHS_WAVES_PER_CU = 8;
-constexpr uint32_t PATHS_TAIL = 1u << 16;
-constexpr bool paths_check(uint32_t bounce) { return bounce == 5 || bounce == 8; }
 
-template <int MODE, bool GEN>
+template <int MODE>
 __global__ __launch_bounds__(TRACE_WG) void k_paths(SceneView sc, const GpuUniforms* __restrict__ U, Planes p,
-                                                    const uint32_t* __restrict__ queue,
-                                                    const uint32_t* __restrict__ count_ptr, Band band) {
+                                                    Band band) {
     __shared__ uint32_t stack_mem[LDS_STACK * TRACE_WG];
     const uint32_t i = blockIdx.x * TRACE_WG + threadIdx.x;
     const GpuUniforms& u = *U;
-    const uint32_t count = GEN ? band.count * u.samples_per_launch : *count_ptr;
-    if (!GEN && count > PATHS_TAIL) return;
     uint32_t visits = 0, tests = 0, overflow = 0, rays = 0, shadow_rays = 0;
-    if (i < count) {
+    if (i < band.count * u.samples_per_launch) {
         RayStack st = make_stack(stack_mem, p.spill, MODE == TRAV_BINARY ? STACK : INST_STACK);
-        const uint32_t pid = GEN ? i : queue[i];
-        const uint32_t pixel = band.first + pid % band.count, sample = u.sample_offset + pid / band.count;
         PathRegs P;
-        if (GEN) {
-            camera_ray(u, pixel, sample, &P.s, &P.origin, &P.dir);
-            P.throughput = v3(1.0f, 1.0f, 1.0f);
-            P.radiance = v3(0.0f, 0.0f, 0.0f);
-            P.prev_position = P.origin;
-            P.prev_bsdf_pdf = 0.0f;
-            P.depth = 0;
-        } else {  // as SHADE reads it
-            const float4 of = p.org[pid], df = p.dir[pid], tf = p.thr[pid], pf = p.prv[pid], rf = p.rad[pid];
-            P.origin = f4xyz(of);
-            P.dir = f4xyz(df);
-            P.throughput = f4xyz(tf);
-            P.radiance = f4xyz(rf);
-            P.prev_position = f4xyz(pf);
-            P.prev_bsdf_pdf = tf.w;
-            P.depth = __float_as_uint(of.w);
-            P.s.sobol = u.sampler_kind == LUCIDA_SAMPLER_SOBOL;
-            P.s.state = __float_as_uint(df.w);
-            P.s.index = sample;
-            P.s.seed = hash_u32(pixel + u.frame_seed * 0x9e3779b9u);
-            P.s.dim = __float_as_uint(pf.w);
-            --rays;  // its first ray is in the queue's own count
-        }
+        camera_ray(u, band.first + i % band.count, u.sample_offset + i / band.count, &P.s, &P.origin, &P.dir);
+        P.throughput = v3(1.0f, 1.0f, 1.0f);
+        P.radiance = v3(0.0f, 0.0f, 0.0f);
+        P.prev_position = P.origin;
+        P.prev_bsdf_pdf = 0.0f;
+        P.depth = 0;
         float4 gal = make_float4(0.0f, 0.0f, 0.0f, 0.0f), gnr = gal;
         for (;;) {
             // EXTEND
@@ -1557,17 +1515,16 @@ __global__ __launch_bounds__(TRACE_WG) void k_paths(SceneView sc, const GpuUnifo
             }
             if (!alive) break;
         }
-        // what RESOLVE reads (the guides are bounce 0's)
-        p.rad[pid] = make_float4(P.radiance.x, P.radiance.y, P.radiance.z, 0.0f);
-        if (GEN) {
-            p.gal[pid] = gal;
-            p.gnr[pid] = gnr;
-        }
+        // what RESOLVE reads
+        p.rad[i] = make_float4(P.radiance.x, P.radiance.y, P.radiance.z, 0.0f);
+        p.gal[i] = gal;
+        p.gnr[i] = gnr;
     }
-    const uint32_t wr = (uint32_t)wave_sum_u32(rays), ws = (uint32_t)wave_sum_u32(shadow_rays);
+    // ray counts into bounce 0's slots (the fold sums every bounce's slot)
+    const uint64_t wr = wave_sum_u32(rays), ws = wave_sum_u32(shadow_rays);
     if ((threadIdx.x & 63) == 0) {
-        if (wr) atomicAdd(&p.counters[PATHS_AT], wr);
-        if (ws) atomicAdd(&p.counters[PATHS_AT + 1], ws);
+        if (wr) atomicAdd(&p.counters[0], (uint32_t)wr);
+        if (ws) atomicAdd(&p.counters[SHADOW_AT], (uint32_t)ws);
     }
     flush_traversal_stats(p.counters, 0u, 0u, overflow, 0u, 0);
 }
@@ -1635,8 +1592,8 @@ __global__ void k_fold_counters(uint32_t* counters, uint32_t depth, uint64_t* ho
     uint64_t* tot = reinterpret_cast<uint64_t*>(counters + TOTALS_AT);
     const uint64_t* batch = reinterpret_cast<const uint64_t*>(counters + STATS_AT);
     uint64_t v[9];
-    v[0] = (lane < depth ? counters[lane] : 0u) + (lane == 0 ? counters[PATHS_AT] : 0u);
-    v[1] = (lane < depth ? counters[SHADOW_AT + lane] : 0u) + (lane == 0 ? counters[PATHS_AT + 1] : 0u);
+    v[0] = lane < depth ? counters[lane] : 0u;
+    v[1] = lane < depth ? counters[SHADOW_AT + lane] : 0u;
     for (int k = 0; k < 7; ++k) v[2 + k] = lane < STATS_STRIPES ? batch[8 * lane + k] : 0u;
     for (int k = 0; k < 9; ++k) {
         for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
@@ -1891,14 +1848,13 @@ static bool binary_width(const lucida_wavefront_config& cfg) { return cfg.bvh_wi
 // EXTEND / CONNECT for the traversal variant `mode` (TRAV_*).
 template <bool BATCH>
 static void launch_extend(int mode, dim3 grid, hipStream_t s, const SceneView& sc, const BatchJob* jobs,
-                          const Planes& p, const uint32_t* queue, const uint32_t* count, uint32_t stats_on,
-                          uint32_t least = 0) {
+                          const Planes& p, const uint32_t* queue, const uint32_t* count, uint32_t stats_on) {
     if (mode == TRAV_INSTANCED)
         hipLaunchKernelGGL((k_extend<BATCH, TRAV_INSTANCED>), grid, dim3(TRACE_WG), 0, s, sc, jobs, p, queue, count,
-                           least, stats_on);
+                           stats_on);
     else
         hipLaunchKernelGGL((k_extend<BATCH, TRAV_BINARY>), grid, dim3(TRACE_WG), 0, s, sc, jobs, p, queue, count,
-                           least, stats_on);
+                           stats_on);
 }
 
 template <bool BATCH>
@@ -2066,13 +2022,11 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
     const uint32_t stats_on = (stats && cfg.count_traversal) ? 1u : 0u;
     const bool profile = stats && cfg.profile_kernels;
 
-    // Renders of few paths trace each path in one launch (k_paths), and instanced
-    // ones of more their last bounces, unless the caller asks for per-stage
-    // times, traversal counts, stages alone or sorted queues.
-    const bool may_paths = !stats_on && !profile && !cfg.serialize && !sort_rays;
-    const bool whole_paths = may_paths && item_paths <= (size_t)ctx->cu_count * PATHS_WAVES_PER_CU * 64;
-    const bool may_tail = may_paths && mode == TRAV_INSTANCED && item_paths >= ((size_t)1 << 18) &&
-                          item_paths < ((size_t)1 << 21);
+    // Renders of few paths trace each path in one launch (k_paths), unless the
+    // caller asks for per-stage times, traversal counts, stages alone or sorted
+    // queues.
+    const bool whole_paths = item_paths <= (size_t)ctx->cu_count * PATHS_WAVES_PER_CU * 64 && !stats_on && !profile &&
+                             !cfg.serialize && !sort_rays;
 
     // Optional per-kernel events: one start/stop pair per launch, destroyed
     // on every return path.
@@ -2118,11 +2072,9 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
         mark(0, true, s);
         const dim3 path_grid(grid_for(Pb, TRACE_WG));
         if (whole_paths && mode == TRAV_INSTANCED)
-            hipLaunchKernelGGL((k_paths<TRAV_INSTANCED, true>), path_grid, dim3(TRACE_WG), 0, s, sc, dU, p, nullptr,
-                               nullptr, it.band);
+            hipLaunchKernelGGL(k_paths<TRAV_INSTANCED>, path_grid, dim3(TRACE_WG), 0, s, sc, dU, p, it.band);
         else if (whole_paths)
-            hipLaunchKernelGGL((k_paths<TRAV_BINARY, true>), path_grid, dim3(TRACE_WG), 0, s, sc, dU, p, nullptr,
-                               nullptr, it.band);
+            hipLaunchKernelGGL(k_paths<TRAV_BINARY>, path_grid, dim3(TRACE_WG), 0, s, sc, dU, p, it.band);
         else
             hipLaunchKernelGGL(k_generate, dim3(grid_for(Pb, 256)), dim3(256), 0, s, dU, p, it.band);
         mark(0, false, s);
@@ -2136,15 +2088,14 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
             uint32_t* qnext = qout;
             uint32_t* order = nullptr;
             mark(1, true, s);
-            const uint32_t least = may_tail && paths_check(b) ? PATHS_TAIL : 0u;
             launch_extend<false>(mode, dim3(grid_for(Pb, TRACE_WG)), s, sc, nullptr, p, qin, p.counters + b,
-                                 stats_on, least);
+                                 stats_on);
             mark(1, false, s);
             if (b > 0) LUCIDA_HIP(hipStreamWaitEvent(s, w.ev_connected, 0), LUCIDA_VALIDATION);
             mark(2, true, s);
             hipLaunchKernelGGL(k_shade<false>, dim3(grid_for(Pb, SHADE_WG)), dim3(SHADE_WG), 0, s, sc, dU, nullptr, p,
                                qin, p.counters + b, qout, p.counters + b + 1, p.counters + SHADOW_AT + b,
-                               sort_rays ? p.qkey : nullptr, it.band, least);
+                               sort_rays ? p.qkey : nullptr, it.band);
             mark(2, false, s);
             LUCIDA_HIP(hipEventRecord(w.ev_shaded, s), LUCIDA_VALIDATION);
             if (sort_rays) {
@@ -2159,11 +2110,6 @@ lucida_status lucida_render_wavefront(lucida_ctx* ctx, const lucida_scene* scene
             launch_connect<false>(mode, dim3(grid_for(Pb, TRACE_WG)), s2, sc, nullptr, p, p.counters + SHADOW_AT + b,
                                   order, stats_on);
             mark(3, false, s2);
-            // a short queue's paths to their ends: after this bounce's CONNECT (both
-            // add to the paths' radiance), before the next SHADE
-            if (may_tail && b + 1 < depth && paths_check(b + 1))
-                hipLaunchKernelGGL((k_paths<TRAV_INSTANCED, false>), dim3(grid_for(PATHS_TAIL, TRACE_WG)),
-                                   dim3(TRACE_WG), 0, s2, sc, dU, p, qnext, p.counters + b + 1, it.band);
             LUCIDA_HIP(hipEventRecord(w.ev_connected, s2), LUCIDA_VALIDATION);
             qin = qnext;
         }
@@ -2528,7 +2474,7 @@ lucida_status lucida_render_batch(lucida_ctx* ctx, const lucida_job* jobs, size_
                     if (b > 0) chk(hipStreamWaitEvent(s, w.ev_connected, 0));
                     hipLaunchKernelGGL(k_shade<false>, dim3(grid_for(P, SHADE_WG)), dim3(SHADE_WG), 0, s, sc, uj,
                                        nullptr, p, qin, p.counters + b, qout, p.counters + b + 1,
-                                       p.counters + SHADOW_AT + b, r.sort ? p.qkey : nullptr, whole, 0u);
+                                       p.counters + SHADOW_AT + b, r.sort ? p.qkey : nullptr, whole);
                     chk(hipEventRecord(w.ev_shaded, s));
                     if (r.sort)
                         chk_sort(sort_queues(w, w.s2, p, qout, P, b, b + 1 < r.depth, RAY_KEY_BITS, &qnext, &order));
@@ -2560,7 +2506,7 @@ lucida_status lucida_render_batch(lucida_ctx* ctx, const lucida_job* jobs, size_
                 if (b > 0) chk(hipStreamWaitEvent(s, w.ev_connected, 0));
                 hipLaunchKernelGGL(k_shade<true>, dim3(grid_for(P, SHADE_WG)), dim3(SHADE_WG), 0, s, none, nullptr, jr,
                                    p, qin, p.counters + b, qout, p.counters + b + 1, p.counters + SHADOW_AT + b,
-                                   r.sort ? p.qkey : nullptr, Band{0u, 0u}, 0u);
+                                   r.sort ? p.qkey : nullptr, Band{0u, 0u});
                 chk(hipEventRecord(w.ev_shaded, s));
                 if (r.sort)
                     chk_sort(sort_queues(w, w.s2, p, qout, P, b, b + 1 < r.depth, 24, &qnext, &order));

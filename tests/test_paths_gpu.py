@@ -1,8 +1,8 @@
 """Renders of few paths, traced a path per thread: the film and the ray counts
 must be those of the wavefront stages, which a render with per-kernel times
 keeps to. Sizes lie on both sides of the path count where one takes over
-(131,072 on 256 CUs), with one batch and several, one bounce and many, and in
-the range (2^18 to 2^21) where instanced scenes' short queues are."""
+(131,072 on 256 CUs), with one batch and several, one bounce and many, and well
+above it, where every render keeps to the stages."""
 from __future__ import annotations
 
 import numpy as np
@@ -17,7 +17,7 @@ CASES = [("box-c1", 1, 1, 1, 8, 0), ("box-c1", 37, 29, 3, 1, 0), ("box-c1", 362,
          ("box-c1", 363, 363, 1, 8, 0), ("cornell-mesh", 512, 256, 1, 8, 0), ("cornell-mesh", 513, 257, 1, 2, 0),
          ("cornell-mesh", 640, 360, 4, 8, 0), ("instances-small", 400, 401, 4, 12, 0),
          ("cornell-mesh", 300, 200, 7, 6, 2), ("instances-small", 96, 64, 9, 12, 4), ("glass-box", 700, 500, 2, 16, 0),
-         # instanced scenes finish short queues from bounces 5 and 8: neither, one or both reached
+         # instanced scenes of 2^18 paths a batch and more, one band and two
          ("instances-small", 640, 512, 2, 12, 0), ("instances-small", 513, 512, 1, 5, 0),
          ("instances-small", 700, 401, 3, 6, 1), ("instance-forest", 800, 600, 4, 16, 0)]
 
