@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "context.hpp"
+#include "film_groups.hpp"
 #include "shading.hpp"
 
 namespace lucida {
@@ -361,8 +362,9 @@ const float4* atrous_enqueue(lucida_ctx* ctx, const lucida_film* const* in, GpuA
     hipStream_t s = ctx->stream;
     size_t base = 0;
     const float4* result = params.iterations % 2 ? pl.b : pl.a;  // the last pass's plane
-    for (size_t first = 0; first < count; first += DN_JOBS) {
-        const unsigned jn = (unsigned)std::min<size_t>(DN_JOBS, count - first);
+    unsigned jn;
+    for (size_t first = 0; first < count; first += jn) {
+        jn = (unsigned)films_together(in + first, count - first, DN_JOBS);
         DnJobs jobs{};
         uint32_t w = 0, h = 0;
         for (unsigned k = 0; k < jn; ++k) {
