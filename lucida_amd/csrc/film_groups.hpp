@@ -15,7 +15,7 @@ constexpr uint64_t EMPTY_PIXELS = 1u << 20;
 // height), from the first on, that go into one launch of at most `most`: as long
 // as the grid stays within twice the films' own pixels and EMPTY_PIXELS. An empty
 // block costs a thirtieth of a full one, but wide and tall films together make
-// any number: of the blocks for 131,072 x 16 and 128 x 16,384 one in 256 had
+// any number: of the blocks for 131,072 x 16 and 128 x 16,384 one in 1,024 had
 // pixels, and a pass over crops of the two took 14.7 ms in shared launches,
 // 0.9 in launches of their own.
 template <class Film>

@@ -804,7 +804,8 @@ size_t net_param_count() {
 
 constexpr size_t CONV_LDS = 160 * 1024 - 512;  // LDS of a CU, less the offset table
 
-template <int MTW, int NT, int PF>
+// Launches k_conv with the epilogue `epi`, one of those that this split serves.
+template <int MTW, int NT, int PF, int... EPI>
 static lucida_status launch_conv_t(hipStream_t s, int epi, ConvArgs a, int wm, int wn) {
     a.wm = wm;
     a.wn = wn;
@@ -815,13 +816,9 @@ static lucida_status launch_conv_t(hipStream_t s, int epi, ConvArgs a, int wm, i
     if (lds > CONV_LDS || wm * wn > 8 || wm * MTW < a.mts || a.in.c_low + a.in.c > CONV_MAX_KBS / 9 * 16)
         return set_error(LUCIDA_INVALID_ARG, "conv: tile larger than a block");
     const dim3 grid(a.n * a.tiles_x * a.tiles_y), block(64 * wm * wn);
-    switch (epi) {
-        case CONV_FWD: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_FWD>), grid, block, lds, s, a); break;
-        case CONV_FWD_POOL: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_FWD_POOL>), grid, block, lds, s, a); break;
-        case CONV_BWD: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_BWD>), grid, block, lds, s, a); break;
-        case CONV_BWD_SPLIT: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_BWD_SPLIT>), grid, block, lds, s, a); break;
-        default: hipLaunchKernelGGL((k_conv<MTW, NT, PF, CONV_BWD_UNPOOL>), grid, block, lds, s, a); break;
-    }
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, lds, s, a); };
+    if (!((epi == EPI && (launch(k_conv<MTW, NT, PF, EPI>), true)) || ...))
+        return set_error(LUCIDA_INVALID_ARG, "conv: no kernel for this split and epilogue");
     return LUCIDA_OK;
 }
 
@@ -839,15 +836,22 @@ static lucida_status launch_conv(hipStream_t s, int epi, const ConvArgs& a) {
     const long px = (long)a.n * a.h * a.w;
     if (mt > 10) return set_error(LUCIDA_INVALID_ARG, "conv: unsupported output channel count");
     if (px < 256L * 256 || mt > 5) {
-        if (px < 128L * 128 && mt <= 8) return launch_conv_t<1, 4, 8>(s, epi, a, mt, 1);
-        return launch_conv_t<2, 4, 4>(s, epi, a, (mt + 1) / 2, mt <= 4 ? 2 : 1);
+        if (px < 128L * 128 && mt <= 8)
+            return launch_conv_t<1, 4, 8, CONV_FWD, CONV_FWD_POOL, CONV_BWD, CONV_BWD_SPLIT, CONV_BWD_UNPOOL>(s, epi, a,
+                                                                                                            mt, 1);
+        return launch_conv_t<2, 4, 4, CONV_FWD, CONV_FWD_POOL, CONV_BWD, CONV_BWD_SPLIT, CONV_BWD_UNPOOL>(
+            s, epi, a, (mt + 1) / 2, mt <= 4 ? 2 : 1);
     }
+    // The concatenations' gradients have 5, 7 and 10 output tiles (layers 12, 10
+    // and 8), the last layer's output one.
     switch (mt) {
-        case 1: return launch_conv_t<1, 8, 4>(s, epi, a, 1, 4);
-        case 2: return a.in.c_low + a.in.c > 64 ? launch_conv_t<2, 4, 4>(s, epi, a, 1, 4) : launch_conv_t<2, 8, 2>(s, epi, a, 1, 4);
-        case 3: return launch_conv_t<3, 4, 4>(s, epi, a, 1, 4);
-        case 4: return launch_conv_t<4, 4, 2>(s, epi, a, 1, 4);
-        default: return launch_conv_t<5, 4, 2>(s, epi, a, 1, 4);
+        case 1: return launch_conv_t<1, 8, 4, CONV_FWD>(s, epi, a, 1, 4);
+        case 2:
+            if (a.in.c_low + a.in.c > 64) return launch_conv_t<2, 4, 4, CONV_FWD>(s, epi, a, 1, 4);
+            return launch_conv_t<2, 8, 2, CONV_FWD, CONV_FWD_POOL, CONV_BWD, CONV_BWD_UNPOOL>(s, epi, a, 1, 4);
+        case 3: return launch_conv_t<3, 4, 4, CONV_FWD, CONV_FWD_POOL, CONV_BWD, CONV_BWD_UNPOOL>(s, epi, a, 1, 4);
+        case 4: return launch_conv_t<4, 4, 2, CONV_FWD, CONV_FWD_POOL, CONV_BWD, CONV_BWD_UNPOOL>(s, epi, a, 1, 4);
+        default: return launch_conv_t<5, 4, 2, CONV_BWD_SPLIT>(s, epi, a, 1, 4);
     }
 }
 
