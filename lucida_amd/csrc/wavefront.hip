@@ -51,7 +51,7 @@ constexpr int MAX_BOUNCES = 64;
 // +64), this batch's traversal counters (u64) at STATS_AT in STATS_STRIPES
 // copies of 8 (a block adds to copy blockIdx % STATS_STRIPES, so the waves
 // of a launch do not queue on a few addresses), the render's running totals
-// (10 u64) at TOTALS_AT.
+// (9 u64) at TOTALS_AT.
 constexpr uint32_t SHADOW_AT = 80;
 constexpr uint32_t STATS_AT = 160;
 constexpr uint32_t STATS_STRIPES = 32;
@@ -1440,14 +1440,18 @@ __global__ __launch_bounds__(TRACE_WG) void k_megakernel(SceneView sc, const Gpu
 // more paths the stages win: they regroup the live paths, and keep up to eight
 // waves on a SIMD where the whole path's registers allow two. The line is what
 // the device holds at once, two waves on each SIMD of its CUs (131,072 paths):
-// up to it a render got faster on every scene, above it slower on most. ms in
-// stages / as paths, at 57,600, 131,044 and 163,840 paths:
-//   box-c1 (10 triangles)      0.40 / 0.21   0.44 / 0.22   0.43 / 0.34
-//   cornell-mesh (10,252)      1.02 / 0.91   1.14 / 1.04   1.12 / 1.25
-//   sphere-c2 (82,944)         1.62 / 1.30   1.76 / 1.31   1.84 / 2.11
-//   sphere-c2 (1,049,844)      2.68 / 1.71   3.00 / 1.79   3.05 / 2.73
-//   instances-c3 (4,096)       5.52 / 4.32   6.04 / 5.01   6.01 / 5.29
-//   bvh-stress (368,640)       1.47 / 1.41   1.73 / 1.52   1.64 / 2.01
+// up to it a render got faster on every scene; a little above it, three of these
+// six still did and three got slower, and the line stays where none does. ms in
+// stages / as paths, at 57,600, 131,044 and 163,840 paths, 8 bounces (instances-c3
+// 12):
+//   box-c1 (10 triangles)      0.35 / 0.18   0.40 / 0.18   0.43 / 0.34
+//   cornell-mesh (10,252)      0.84 / 0.75   0.92 / 0.75   1.12 / 1.25
+//   sphere-c2 (82,944)         1.62 / 1.23   1.74 / 1.30   1.84 / 2.11
+//   sphere-c2 (1,049,844)      2.56 / 1.70   2.91 / 1.75   3.05 / 2.73
+//   instances-c3 (4,096)       5.74 / 4.67   6.03 / 4.67   6.01 / 5.29
+//   bvh-stress (368,640)       1.50 / 1.41   1.59 / 1.50   1.64 / 2.01
+// Batches of up to that many paths, eight of them in two pipelines: 0.99 (bvh-stress)
+// to 4.1 times as fast as in stages, 1.02 and more on every other scene.
 // ---------------------------------------------------------------------------
 constexpr size_t PATHS_WAVES_PER_CU = 8;
 
