@@ -89,3 +89,24 @@ def test_tiles_equal_the_untiled_passes(gpu, iterations, sigmas):
     same = slice(0, h - reach)
     assert np.isfinite(tiled).all()
     np.testing.assert_array_equal(tiled[same].view(np.uint32), untiled[same].view(np.uint32))
+
+
+@pytest.mark.parametrize("sigmas", [(64.0, -4.0e-39, 4.0, 0.1), (64.0, 0.08, -40.0, 0.1), (64.0, 0.08, 4.0, -1.0)],
+                         ids=["depth", "luminance", "albedo"])
+def test_stops_that_are_not_positive(gpu, oracle, sigmas):
+    """They are accepted and take the untiled passes: as part of a tile a pixel
+    outside the film could get a weight (the depth stop's term there, 10 over
+    -4e-38, is infinite, where every pixel of this film has none). One surface
+    of one depth and albedo, so the taps' weights are the kernel's times the
+    luminance stop's; bounds as for films of any kind: a weight off by 2e-5 of
+    itself, a pass's mean by twice that of the largest colour."""
+    w, h = 20, 13
+    print(f"a-trous case {w}x{h}, stops {sigmas}", flush=True)
+    acc = plain_film(w, h, 1.0, 3)
+    acc["depth"] = 10.0
+    p = L.DenoiseParams(4, *sigmas)
+    got = filtered(gpu, acc, w, h, p)
+    a = as_float16(acc).reshape(h, w, 16)
+    want = oracle.denoise(a[..., 0:3], a[..., 4:7], a[..., 8:11], a[..., 7], p)
+    assert np.isfinite(want).all() and np.abs(want - a[..., 0:3]).max() > 0.1
+    assert np.abs(got[..., 0:3] - want).max() <= 5e-4 * np.abs(want).max()
